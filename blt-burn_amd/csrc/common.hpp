@@ -205,6 +205,12 @@ __device__ inline int wave_max_i32(int v) {
   return max((int)s32[0], (int)s32[1]);
 }
 
+// RMSNorm factor (eps after the root, model.rs:758-770) of a row from its sum
+// of squares; every kernel that forms one uses this expression.
+__device__ inline float row_factor(float ss, int dim, float eps) {
+  return 1.f / (sqrtf(ss / (float)dim) + eps);
+}
+
 inline unsigned ceil_div(int64_t a, int64_t b) { return (unsigned)((a + b - 1) / b); }
 
 // Wait until at most N of this wave's vector-memory loads are outstanding and

@@ -4,12 +4,13 @@
 // store, in-place f32 residual add, RoPE on the q/k columns of the fused QKV
 // projection, SiLU*gate of the fused W1|W3 FFN).
 //
-// Two kernels share the tiling and the epilogue layout:
+// Three kernels share the tiling and the epilogue layout:
 // gemm_bf16_dma_persistent_kernel (global -> LDS by DMA, 256 x 256 x 64 tiles
-// with one persistent block per CU, or 128 x 128 x 64 tiles with two for
-// launches that have fewer 256 x 256 tiles than CUs; LDS-staged epilogue; every
-// projection of the model, N % 256 == 0) and gemm_bf16_kernel (register-staged
-// loads; any N, e.g. the 260-wide head).
+// with one persistent block per CU, LDS-staged epilogue; N % 256 == 0 and
+// enough rows), gemm_bf16_pipe_kernel (the same on smaller tiles with loader
+// waves and deeper stages, one block per tile: launches that 256 x 256 tiles
+// would not fill the chip with) and gemm_bf16_kernel (register-staged loads;
+// any N, e.g. the 260-wide head).
 //
 // Tiling: a BM x BN block tile is split over WM x WN wave64s; each wave owns a
 // (BM/WM) x (BN/WN) tile made of 32x32 v_mfma_f32_32x32x16_bf16 sub-tiles,
@@ -406,13 +407,46 @@ __device__ inline void load_rope_cs(const GemmArgs& p, int64_t row, int lane, f3
   }
 }
 
+// The residual epilogue's global inputs of one wave tile: 32-row slab i's
+// residual pieces (lane's pieces lane + 64 t of the slab's 16-byte pieces) and
+// the consumer's norm weight for the lane's 4 columns (the same columns in
+// every slab), applied to the bf16 copy only.  Rows row0 + r and columns col0
+// + c exist for r < mrem, c < nrem (both > 0); pieces out of range read the
+// last row or column and are not stored.
+template <class C>
+struct ResidIn {
+  static constexpr int CPR = C::WTN / 4;    // 16-byte pieces per row
+  static constexpr int NP = 32 * CPR / 64;  // pieces per lane per 32-row slab
+  f32x4_t res[NP];
+  f32x4_t csc;
+  // cb: the f32 residual at (row0, col0)
+  __device__ inline void load_slab(const char* cb, int i, int lane, int mrem, int nrem, int ldc) {
+#pragma unroll
+    for (int t = 0; t < NP; ++t) {
+      const int q = lane + 64 * t, r = i * 32 + q / CPR, c = (q % CPR) * 4;
+      const int rr = r < mrem ? r : mrem - 1;
+      const int cc = c < nrem ? c : nrem - 4;
+      res[t] = *reinterpret_cast<const f32x4_t*>(cb + (unsigned)((rr * ldc + cc) * 4));
+    }
+  }
+  __device__ inline void load_scale(const GemmArgs& p, int64_t col0, int lane, int nrem) {
+    csc = f32x4_t{1.f, 1.f, 1.f, 1.f};
+    if (p.col_scale) {
+      const int c = (lane % CPR) * 4;
+      csc = *reinterpret_cast<const f32x4_t*>(p.col_scale + col0 + (c < nrem ? c : nrem - 4));
+    }
+  }
+};
+
 // cs0: the table pairs of the lane's first row block, loaded by the caller
-// ahead of time (QKV only).
-template <class C, int EPI>
+// ahead of time (QKV only).  PRE: rin holds slab 0's residual pieces and the
+// column scale, loaded by the caller ahead of time (residual epilogue only).
+// NT: bf16 outputs are stored non-temporally.
+template <class C, int EPI, bool PRE, bool NT>
 __device__ inline void epilogue_lds(const GemmArgs& p, f32x16_t (&acc)[C::TM][C::TN], int64_t m0,
                                     int64_t n0, int wid, int wm, int wn, int lane,
                                     unsigned char* smem, const float (&rs)[C::TM],
-                                    const f32x4_t (&cs0)[8]) {
+                                    const f32x4_t (&cs0)[8], ResidIn<C>& rin) {
   const int lrow = lane & 31, lhalf = lane >> 5;
   const int64_t row0 = m0 + wm * C::WTM;  // first row of this wave's tile
   const int64_t col0 = n0 + wn * C::WTN;  // first column (pre-epilogue index)
@@ -438,23 +472,9 @@ __device__ inline void epilogue_lds(const GemmArgs& p, f32x16_t (&acc)[C::TM][C:
     // Residual pieces: slab i + 1's are loaded as soon as slab i's have been
     // added, so their latency overlaps slab i's stores and slab i + 1's
     // staging (one buffer: the 8-wave kernels have no registers for two).
-    f32x4_t res[NP];
-    auto load_resid = [&](int i) {
-#pragma unroll
-      for (int t = 0; t < NP; ++t) {
-        const int q = lane + 64 * t, r = i * 32 + q / CPR, c = (q % CPR) * 4;
-        const int rr = r < mrem ? r : mrem - 1;  // out-of-range pieces are not stored
-        const int cc = c < nrem ? c : nrem - 4;
-        res[t] = *reinterpret_cast<const f32x4_t*>(cb + (unsigned)((rr * ldc + cc) * 4));
-      }
-    };
-    if (resid) load_resid(0);
-    // the consumer's norm weight for this lane's 4 columns (the same columns
-    // in every slab: 64 | 64 * t), applied to the bf16 copy only
-    f32x4_t csc = f32x4_t{1.f, 1.f, 1.f, 1.f};
-    if (resid && p.col_scale) {
-      const int c = (lane % CPR) * 4;
-      csc = *reinterpret_cast<const f32x4_t*>(p.col_scale + col0 + (c < nrem ? c : nrem - 4));
+    if (resid && !PRE) {
+      rin.load_slab(cb, 0, lane, mrem, nrem, ldc);
+      rin.load_scale(p, col0, lane, nrem);
     }
 #pragma unroll
     for (int i = 0; i < C::TM; ++i) {
@@ -473,9 +493,9 @@ __device__ inline void epilogue_lds(const GemmArgs& p, f32x16_t (&acc)[C::TM][C:
         const int q = lane + 64 * t, r = q / CPR, c = q % CPR;
         const float* sp = buf + r * LD + c * 4;
         v[t] = f32x4_t{sp[0], sp[1], sp[2], sp[3]};
-        if (resid) v[t] += res[t];
+        if (resid) v[t] += rin.res[t];
       }
-      if (resid && i + 1 < C::TM) load_resid(i + 1);
+      if (resid && i + 1 < C::TM) rin.load_slab(cb, i + 1, lane, mrem, nrem, ldc);
 #pragma unroll
       for (int t = 0; t < NP; ++t) {
         const int q = lane + 64 * t, r = i * 32 + q / CPR, c = (q % CPR) * 4;
@@ -487,7 +507,7 @@ __device__ inline void epilogue_lds(const GemmArgs& p, f32x16_t (&acc)[C::TM][C:
           if (resid) {
             *reinterpret_cast<f32x4_t*>(o) = v[t];
             if (xbb) {
-              const f32x4_t y = v[t] * csc;
+              const f32x4_t y = v[t] * rin.csc;
               *reinterpret_cast<u32x2_t*>(xbb + off * 2u) =
                   u32x2_t{pack_bf16x2(y.x, y.y), pack_bf16x2(y.z, y.w)};
               ss = v[t].x * v[t].x + v[t].y * v[t].y + v[t].z * v[t].z + v[t].w * v[t].w;
@@ -516,7 +536,8 @@ __device__ inline void epilogue_lds(const GemmArgs& p, f32x16_t (&acc)[C::TM][C:
   // rope_cols % 64 == 0: each 64-column head is rotated or not as a whole
   const bool rope = EPI == EPI_QKV_ROPE && col0 < p.rope_cols;
   constexpr int LD = C::WTN + 4;  // bf16 row pitch (8-byte pad)
-  uint16_t* buf = reinterpret_cast<uint16_t*>(smem) + wid * 64 * LD;
+  constexpr int SLAB = C::TM > 1 ? 2 : 1;  // 32-row blocks per staged slab
+  uint16_t* buf = reinterpret_cast<uint16_t*>(smem) + wid * 32 * SLAB * LD;
   // RoPE (cos, sin) pairs of this lane's 16 frequencies (8 g + 4 lhalf + e)
   // for its row of tile row i, loaded one row ahead
   f32x4_t cscur[8], csnext[8];
@@ -526,11 +547,11 @@ __device__ inline void epilogue_lds(const GemmArgs& p, f32x16_t (&acc)[C::TM][C:
     for (int t = 0; t < 8; ++t) csnext[t] = cs0[t];
   }
 #pragma unroll
-  for (int i0 = 0; i0 < C::TM; i0 += 2) {
+  for (int i0 = 0; i0 < C::TM; i0 += SLAB) {
 #pragma unroll
-    for (int ii = 0; ii < 2; ++ii) {
+    for (int ii = 0; ii < SLAB; ++ii) {
       const int i = i0 + ii;
-      const int rl = ii * 32 + lrow;  // row within this 64-row slab
+      const int rl = ii * 32 + lrow;  // row within this slab
       if constexpr (EPI == EPI_BF16) {
 #pragma unroll
         for (int j = 0; j < C::TN; ++j)
@@ -602,23 +623,26 @@ __device__ inline void epilogue_lds(const GemmArgs& p, f32x16_t (&acc)[C::TM][C:
         }
     }
     wave_lds_fence();
-    // stream the 64-row slab out: OW columns per row in 16-byte pieces
+    // stream the slab out: OW columns per row in 16-byte pieces
     const int OW = silu ? C::WTN / 2 : C::WTN;
     const int CPR = OW / 8;
     const int64_t ocol0 = silu ? col0 / 2 : col0;
-    for (int q = lane; q < 64 * CPR; q += 64) {
+    for (int q = lane; q < 32 * SLAB * CPR; q += 64) {
       const int r = q / CPR, c = q % CPR;
       const int64_t row = row0 + i0 * 32 + r;
       const uint16_t* sp = buf + r * LD + c * 8;
       const u32x2_t lo = *reinterpret_cast<const u32x2_t*>(sp);
       const u32x2_t hi = *reinterpret_cast<const u32x2_t*>(sp + 4);
-      // non-temporal: the tile's output is not read again by this launch, and
-      // the next kernel's reads of it (the whole output exceeds the MALL) come
-      // from HBM either way; every CU stores its slab at the same time here
-      if (row < p.M)
-        __builtin_nontemporal_store(u32x4_t{lo.x, lo.y, hi.x, hi.y},
-                                    reinterpret_cast<u32x4_t*>(reinterpret_cast<uint16_t*>(p.C) +
-                                                               row * p.ldc + ocol0 + c * 8));
+      const u32x4_t w = u32x4_t{lo.x, lo.y, hi.x, hi.y};
+      u32x4_t* o = reinterpret_cast<u32x4_t*>(reinterpret_cast<uint16_t*>(p.C) + row * p.ldc +
+                                              ocol0 + c * 8);
+      // non-temporal where the whole output exceeds the MALL (the next kernel
+      // reads it from HBM either way, and every CU stores its slab at the
+      // same time here); a small launch's output stays cached for its reader
+      if (row < p.M) {
+        if constexpr (NT) __builtin_nontemporal_store(w, o);
+        else *o = w;
+      }
     }
     wave_lds_fence();
   }
@@ -627,9 +651,8 @@ __device__ inline void epilogue_lds(const GemmArgs& p, f32x16_t (&acc)[C::TM][C:
 
 // Same tiling and epilogues as gemm_bf16_kernel, but K tiles move global ->
 // LDS by the LDS-DMA path (no VGPR staging, no ds_write) through two LDS
-// stages, and the kernel is persistent: each resident block (one per CU on
-// 256 x 256 tiles, two on 128 x 128) walks the tiles v = blockIdx.x,
-// blockIdx.x + gridDim.x, ...  With gridDim.x a multiple of 8
+// stages, and the kernel is persistent: each resident block (one per CU)
+// walks the tiles v = blockIdx.x, blockIdx.x + gridDim.x, ...  With gridDim.x a multiple of 8
 // every tile of a block has the block's XCD residue, so the tile order of
 // tile_origin holds.  The K-tile stream runs on across tiles: the next tile's
 // first K tile is issued together with the current tile's last one, so its
@@ -789,7 +812,9 @@ void gemm_bf16_dma_persistent_kernel(GemmArgs p) {
     // the loop (hoisted out, it would occupy registers through the K loop)
     int le = lane;
     asm volatile("" : "+v"(le));
-    epilogue_lds<C, EPI>(p, acc, m0, n0, wid, wm, wn, le, lds + (st == 0 ? SB : 0), rs, cs0);
+    ResidIn<C> rin;
+    epilogue_lds<C, EPI, false, true>(p, acc, m0, n0, wid, wm, wn, le, lds + (st == 0 ? SB : 0),
+                                      rs, cs0, rin);
     if (!more) break;
     v = vn;
     m0 = m0n;
@@ -804,6 +829,207 @@ void gemm_bf16_dma_persistent_kernel(GemmArgs p) {
     // the epilogue's LDS
     dma_wait_barrier<0>();
   }
+}
+
+// The row factors of a consumer that forms them itself: the norm partials of
+// this lane's rows (p.row_np of them, a multiple of 4 up to 16) are loaded
+// before the K loop, and finish() sums them after it in row_rstd_kernel's
+// order, so the factors equal that kernel's bit for bit.
+template <class C>
+struct RowNorms {
+  f32x4_t s[C::TM][4];
+  __device__ inline void load(const GemmArgs& p, int64_t row0) {
+#pragma unroll
+    for (int i = 0; i < C::TM; ++i) {
+      const int64_t r = row0 + i * 32;
+      const float* src = p.row_ss + (r < p.M ? r : p.M - 1) * p.row_np;
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        if (4 * q < p.row_np) s[i][q] = *reinterpret_cast<const f32x4_t*>(src + 4 * q);
+    }
+  }
+  __device__ inline void finish(const GemmArgs& p, float (&rs)[C::TM]) const {
+#pragma unroll
+    for (int i = 0; i < C::TM; ++i) {
+      float t = 0.f;
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        if (4 * q < p.row_np) {
+          t += s[i][q].x;
+          t += s[i][q].y;
+          t += s[i][q].z;
+          t += s[i][q].w;
+        }
+      rs[i] = row_factor(t, p.row_dim, p.row_eps);
+    }
+  }
+};
+
+// Launches that do not fill the chip with 256 x 256 tiles: one block per BM x
+// BN tile, WM x WN MFMA waves and NL loader waves.  The loaders keep S - 1 K
+// tiles of 64 in flight by LDS DMA; one block barrier per K tile hands a
+// landed tile to the MFMA waves and the stage they have read back to the
+// loaders.
+//
+// What bounds it: the latency of a serial K walk with one or two blocks per
+// CU, not bandwidth or the matrix cores.  Timing copies of the 64 x 64 tile on
+// M = 48, N = 768, K = 2048 (an empty kernel takes 2.2 us): waits and barriers
+// alone 44 ns per K tile, the DMA issue 81 ns, fragment reads and MFMAs 170 ns,
+// and in one set of waves these add (11.8 us; deeper stages, the DMA spread
+// over the K steps and fragment reads ahead of the barrier changed nothing).
+// With the DMA in waves of its own the launch takes 9.6 us, against 24 us for
+// the two-stage persistent kernel on 128 x 128 tiles, whose every K tile waits
+// for the one load in flight.  For the same reason the epilogue's global inputs
+// (row factors or norm partials, the residual, the RoPE pairs) are requested
+// before the K loop.
+//
+// The wave tile keeps its 64 columns, the K order per output (from the last
+// tile down where the first column has bit 10 set) and the per-64-column norm
+// partials, so every output is bit-identical to the 256 x 256 launch's.
+template <int BM, int BN, int WM, int WN, int NL, int S, int EPI>
+__global__ __launch_bounds__(64 * (WM * WN + NL)) void gemm_bf16_pipe_kernel(GemmArgs p) {
+  constexpr int BK = 64;
+  using C = GemmCfg<BM, BN, BK, WM, WN>;
+  constexpr int NW = WM * WN;
+  constexpr int RPC = 64 / C::CH;          // LDS rows per 1-KB DMA chunk
+  constexpr int RPB = 128 / BK;            // rows per 256 bytes (swizzle period)
+  constexpr int QA = BM / RPC / NL;        // chunks per loader wave per stage: A rows,
+  constexpr int QB = BN / RPC / NL;        // then Bt rows
+  constexpr int NI = QA + QB;
+  constexpr int SB = C::STAGE * 2;         // bytes per stage
+  static_assert(BM % (RPC * NL) == 0 && BN % (RPC * NL) == 0, "chunks divide over the loaders");
+  static_assert(NI * (S - 2) <= 63, "outstanding DMA must fit the vmcnt field");
+  constexpr int SLAB = C::TM > 1 ? 2 : 1;
+  static_assert(NW * 32 * SLAB * (C::WTN + 4) * 2 <= S * SB && NW * 32 * (C::WTN + 2) * 4 <= S * SB,
+                "staged epilogue must fit in the stages");
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[S * SB];
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform (SGPR)
+  int64_t m0, n0;
+  tile_origin<BM, BN>(p, blockIdx.x, m0, n0);
+  const int KT = (int)(p.K / BK);
+
+  if (wid >= NW) {
+    // ---- loader wave ----
+    const int lw = wid - NW;
+    const unsigned lds_base = (unsigned)(uintptr_t)lds;
+    const bool rev = (n0 >> 10) & 1;
+    // chunk q covers operand rows (q NL + lw) RPC ..; rows past the operand
+    // read its last row, whose results are never stored
+    unsigned goff[NI];
+#pragma unroll
+    for (int q = 0; q < NI; ++q) {
+      const bool isA = q < QA;
+      const int r = ((isA ? q : q - QA) * NL + lw) * RPC + lane / C::CH;
+      const int c = (lane % C::CH) ^ ((r / RPB) & (C::CH - 1));
+      const int64_t last = isA ? p.M - 1 - m0 : p.N - 1 - n0;
+      goff[q] = (unsigned)(((r < last ? r : last) * (isA ? p.lda : p.ldb) + c * 8) * 2);
+    }
+    const uint16_t* abase = p.A + m0 * p.lda;
+    const uint16_t* bbase = p.Bt + n0 * p.ldb;
+    // t-th K tile in this block's order, into stage st
+    auto dma_tile = [&](int t, int st) {
+      const int64_t k0 = (int64_t)(rev ? KT - 1 - t : t) * BK;
+      const unsigned sbase = lds_base + (unsigned)(st * SB);
+#pragma unroll
+      for (int q = 0; q < NI; ++q) {
+        const bool isA = q < QA;
+        const unsigned row = (unsigned)(((isA ? q : q - QA) * NL + lw) * RPC);
+        dma16_so((isA ? abase : bbase) + k0, goff[q],
+                 sbase + (isA ? 0u : (unsigned)(BM * BK * 2)) + row * (unsigned)(BK * 2));
+      }
+    };
+    // waits until at most `newer` of this wave's tiles are in flight
+    // (newer <= S - 2), then joins the block barrier
+    auto wait_tile = [&](int newer) {
+      static_for<0, S - 1>([&](auto n) {
+        if (newer == decltype(n)::value) dma_wait_barrier<NI * decltype(n)::value>();
+      });
+    };
+#pragma unroll
+    for (int t = 0; t < S - 1; ++t)
+      if (t < KT) dma_tile(t, t);
+    int stn = S - 1;
+    for (int t = 0; t < KT; ++t) {
+      // tile t has landed; past the barrier every MFMA wave has read tile
+      // t - 1, whose stage takes tile t + S - 1
+      wait_tile(KT - 1 - t < S - 2 ? KT - 1 - t : S - 2);
+      if (t + S - 1 < KT) dma_tile(t + S - 1, stn);
+      stn = stn + 1 < S ? stn + 1 : 0;
+    }
+    asm volatile("s_barrier" ::: "memory");
+    return;
+  }
+
+  // ---- MFMA wave ----
+  const int wm = wid / WN, wn = wid % WN;
+  const int lrow = lane & 31, lhalf = lane >> 5;
+  // the epilogue's global inputs, requested ahead of the K loop
+  const int64_t row0 = m0 + wm * C::WTM, col0 = n0 + wn * C::WTN;
+  float rs[C::TM];
+  RowNorms<C> rn;
+  if (p.row_ss) rn.load(p, row0 + lrow);
+  else load_row_scales<C>(p, row0 + lrow, rs);
+  // (two 32-row blocks per wave have no registers for the residual and the
+  // RoPE pairs through the K loop: they load them after it)
+  constexpr bool PRE = C::TM == 1;
+  f32x4_t cs0[8];
+  const bool rope = EPI == EPI_QKV_ROPE && col0 < p.rope_cols;
+  if (PRE && rope) load_rope_cs(p, row0 + lrow, lane, cs0);
+  ResidIn<C> rin;
+  if (PRE && EPI == EPI_RESID_F32 && row0 < p.M && col0 < p.N) {
+    const int mrem = (int)(p.M - row0 < C::WTM ? p.M - row0 : C::WTM);
+    const int nrem = (int)(p.N - col0 < C::WTN ? p.N - col0 : C::WTN);
+    rin.load_slab(reinterpret_cast<const char*>(reinterpret_cast<const float*>(p.C) +
+                                                row0 * p.ldc + col0),
+                  0, lane, mrem, nrem, (int)p.ldc);
+    rin.load_scale(p, col0, lane, nrem);
+  }
+  f32x16_t acc[C::TM][C::TN];
+#pragma unroll
+  for (int i = 0; i < C::TM; ++i)
+#pragma unroll
+    for (int j = 0; j < C::TN; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+  auto load_frags = [&](int st, int ks, bf16x8_t (&af)[C::TM], bf16x8_t (&bfr)[C::TN]) {
+    const uint16_t* sa = reinterpret_cast<const uint16_t*>(lds + st * SB);
+    const uint16_t* sb = sa + BM * BK;
+    const int chunk = ks * 2 + lhalf;
+#pragma unroll
+    for (int i = 0; i < C::TM; ++i)
+      af[i] = *reinterpret_cast<const bf16x8_t*>(sa + swz<BK>(wm * C::WTM + i * 32 + lrow, chunk));
+#pragma unroll
+    for (int j = 0; j < C::TN; ++j)
+      bfr[j] = *reinterpret_cast<const bf16x8_t*>(sb + swz<BK>(wn * C::WTN + j * 32 + lrow, chunk));
+  };
+  // this wave's LDS reads are done, and after the barrier every wave's are
+  auto lds_barrier = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+  bf16x8_t af[2][C::TM], bfr[2][C::TN];
+  int st = 0;  // stage of K tile t
+  for (int t = 0; t < KT; ++t) {
+    lds_barrier();
+    // fragments of K step ks + 1 are read beside the MFMAs of step ks
+    load_frags(st, 0, af[0], bfr[0]);
+    static_for<0, BK / 16>([&](auto kc) {
+      constexpr int ks = decltype(kc)::value;
+      if constexpr (ks + 1 < BK / 16) load_frags(st, ks + 1, af[(ks + 1) & 1], bfr[(ks + 1) & 1]);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < C::TM; ++i)
+#pragma unroll
+        for (int j = 0; j < C::TN; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bfr[ks & 1][j], af[ks & 1][i],
+                                                              acc[i][j], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    st = st + 1 < S ? st + 1 : 0;
+  }
+  if (!PRE && rope) load_rope_cs(p, row0 + lrow, lane, cs0);
+  if (p.row_ss) rn.finish(p, rs);
+  lds_barrier();
+  epilogue_lds<C, EPI, PRE, false>(p, acc, m0, n0, wid, wm, wn, lane, lds, rs, cs0, rin);
 }
 
 }  // namespace gemm

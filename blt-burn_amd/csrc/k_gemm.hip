@@ -20,10 +20,9 @@ int device_cus() {
 template <int BM, int BN, int BK, int WM, int WN, int EPI>
 int run_gemm_persistent(const GemmArgs& a, hipStream_t s) {
   const int64_t nb = ((a.M + BM - 1) / BM) * ((a.N + BN - 1) / BN);
-  // as many blocks as fit on the CUs at once (256x256: one per CU, its LDS
-  // holds 160 KB; 128x128: two, 80 KB each), a multiple of 8 blocks so each
+  // one block per CU (its LDS holds 160 KB), a multiple of 8 blocks so each
   // keeps its XCD residue
-  int64_t grid = (int64_t)device_cus() * (BM * BN <= 128 * 128 ? 2 : 1);
+  int64_t grid = device_cus();
   grid = grid >= 8 ? grid & ~7 : grid;
   if (grid <= 0 || grid > nb) grid = nb;
   hipLaunchKernelGGL((gemm::gemm_bf16_dma_persistent_kernel<BM, BN, BK, WM, WN, EPI>),
@@ -45,6 +44,87 @@ int run_gemm_dma_epi(const GemmArgs& a, hipStream_t s) {
   return fail(-2, "gemm: unknown epilogue");
 }
 
+template <int BM, int BN, int WM, int WN, int NL, int S, int EPI>
+int run_gemm_pipe(const GemmArgs& a, hipStream_t s) {
+  const int64_t nb = ((a.M + BM - 1) / BM) * ((a.N + BN - 1) / BN);
+  hipLaunchKernelGGL((gemm::gemm_bf16_pipe_kernel<BM, BN, WM, WN, NL, S, EPI>),
+                     dim3((unsigned)nb), dim3(64 * (WM * WN + NL)), 0, s, a);
+  BLT_LAUNCH_CHECK("gemm_bf16_pipe_kernel");
+  return 0;
+}
+
+template <int BM, int BN, int WM, int WN, int NL, int S>
+int run_gemm_pipe_epi(GemmArgs a, hipStream_t s) {
+  // tile groups of 1024 rows: their A rows (1.5 MB at K = 768) stay in an XCD's
+  // L2 while it walks the columns.  N <= 1024 with at least as many rows: N
+  // fastest (its whole Bt is what stays).
+  a.group_m = a.N > 1024 || a.M < a.N ? 1024 / BM : 0;
+  switch (a.epi) {
+    case EPI_BF16: return run_gemm_pipe<BM, BN, WM, WN, NL, S, EPI_BF16>(a, s);
+    case EPI_F32: return run_gemm_pipe<BM, BN, WM, WN, NL, S, EPI_F32>(a, s);
+    case EPI_RESID_F32: return run_gemm_pipe<BM, BN, WM, WN, NL, S, EPI_RESID_F32>(a, s);
+    case EPI_QKV_ROPE: return run_gemm_pipe<BM, BN, WM, WN, NL, S, EPI_QKV_ROPE>(a, s);
+    case EPI_SILU_GATE: return run_gemm_pipe<BM, BN, WM, WN, NL, S, EPI_SILU_GATE>(a, s);
+  }
+  return fail(-2, "gemm: unknown epilogue");
+}
+
+// ---- choice of the tile (N % 256 == 0) ---------------------------------------
+// The predicted time of a launch on each tile, in us, with n tiles, c = ceil(n /
+// CUs) of them on the fullest CU and KT K tiles:
+//   fix + c (k KT + e) + (n / CUs) (kf KT + r)
+// e per tile for the epilogue of its class (residual, other), the last term the
+// memory traffic that grows with the whole launch (r: the residual's).  The
+// constants are least-squares fits to the measured times of the four projection
+// shapes of the model (N, K = 2304, 768; 768, 768; 4096, 768; 768, 2048) at M = 48
+// .. 40000; over those 72 launches the tile it picks is within 8 % of the best of
+// eleven tried (mean 0.8 %).  Measured us (256 x 256 | picked), N = 768, K =
+// 2048: M = 48: 45.5 | 9.6 (64 x 64); 1536: 49.8 | 13.1 (64 x 128); 4096: 50.1 |
+// 20.1 (128 x 128); 8192: 52.4 | 32.4 (128 x 256); 40000: 143 | 143 (128 x 256: 154).
+// All tiles give bit-identical results, so the choice is free of M.
+enum Tile { T64x64, T64x128, T128x128, T128x256, T256x256 };
+struct TileCost {
+  int bm, bn;
+  double fix, k, e_resid, e_other, kf, r;
+};
+constexpr TileCost kTileCost[] = {
+    {64, 64, 4.393, 0.164, 0.036, 0.422, 0.011, 0.841},
+    {64, 128, 3.267, 0.269, 0.075, 0.626, 0.004, 1.774},
+    {128, 128, 1.160, 0.341, 2.711, 3.454, 0.078, 4.828},
+    {128, 256, 1.039, 0.533, 5.597, 5.132, 0.212, 5.656},
+    {256, 256, 2.580, 1.167, 6.264, 6.274, 0.308, 11.024},
+};
+Tile pick_tile(int64_t M, int64_t N, int64_t K, bool resid) {
+  const int cus = device_cus() > 0 ? device_cus() : 256;
+  const double KT = (double)(K / 64);
+  const int64_t nb256 = ((M + 255) / 256) * (N / 256);
+  if (nb256 >= 8 * (int64_t)cus) return T256x256;  // its rounds fill the chip
+  double best = 0;
+  Tile t = T256x256;
+  for (int i = 0; i < 5; ++i) {
+    const TileCost& w = kTileCost[i];
+    const int64_t n = ((M + w.bm - 1) / w.bm) * ((N + w.bn - 1) / w.bn);
+    const double c = (double)((n + cus - 1) / cus), f = (double)n / cus;
+    double est = w.fix + c * (w.k * KT + (resid ? w.e_resid : w.e_other)) +
+                 f * (w.kf * KT + (resid ? w.r : 0.0));
+    // a full chip of 256 x 256 tiles moves the fewest operand bytes: leave it
+    // only for a clear gain
+    if (i == T256x256 && nb256 >= cus) est *= 0.95;
+    if (i == 0 || est < best) {
+      best = est;
+      t = (Tile)i;
+    }
+  }
+  return t;
+}
+
+// a 256-row tile's operand and output rows are addressed with 32-bit byte
+// offsets, so their reach must fit
+bool tile_reach_fits(const GemmArgs& a) {
+  const int64_t two31 = int64_t(1) << 31;
+  return 256 * (a.lda > a.ldb ? a.lda : a.ldb) * 2 + a.K * 2 < two31 && 256 * a.ldc * 4 < two31;
+}
+
 template <int BM, int BN, int BK, int WM, int WN, int PF, int OCC>
 int run_gemm(const GemmArgs& a, hipStream_t s) {
   const int64_t nb = ((a.M + BM - 1) / BM) * ((a.N + BN - 1) / BN);
@@ -55,6 +135,12 @@ int run_gemm(const GemmArgs& a, hipStream_t s) {
 }
 
 }  // namespace
+
+// (dense operands: the model's launches)
+bool gemm_takes_norm_partials(int64_t M, int64_t N, int64_t K, int np) {
+  return np % 4 == 0 && np <= 16 && N % 256 == 0 && K * 512 + K * 2 < (int64_t(1) << 31) &&
+         N * 1024 < (int64_t(1) << 31) && pick_tile(M, N, K, false) != T256x256;
+}
 
 int launch_gemm(const GemmArgs& a_in, hipStream_t s) {
   GemmArgs a = a_in;
@@ -76,27 +162,26 @@ int launch_gemm(const GemmArgs& a_in, hipStream_t s) {
 
   if ((uintptr_t)a.A % 16 != 0 || (uintptr_t)a.Bt % 16 != 0 || a.lda % 8 != 0 || a.ldb % 8 != 0)
     return fail(-2, "gemm: A and Bt rows must be 16-byte aligned (lda, ldb % 8 == 0)");
+  if (a.row_ss && (a.row_np % 4 != 0 || a.row_np > 16 || (uintptr_t)a.row_ss % 16 != 0))
+    return fail(-2, "gemm: row_ss needs row_np % 4 == 0, row_np <= 16, 16-byte alignment");
   // Wide N (QKV, W1|W3): walk groups of 8 M-tiles so the blocks resident on
   // an XCD share A and Bt tiles in its L2; narrow N (O, W2: 3 tiles): N fastest.
   a.group_m = (a.N + 255) / 256 >= 8 ? 8 : 0;
-  // N % 256 == 0: persistent 256x256 tiles over 8 waves (wave tile 128x64),
-  // K tiles of 64 moved by LDS DMA through 2 stages, LDS-staged epilogue; it
-  // addresses a tile's operand and output rows with 32-bit byte offsets, so
-  // their reach must fit.  Otherwise (the 260-wide head, huge strides)
+  // N % 256 == 0: K tiles of 64 moved by LDS DMA, LDS-staged epilogue, on the
+  // tile pick_tile chooses.  Otherwise (the 260-wide head, huge strides)
   // 128x128 register-staged tiles over 4 waves.
-  const int64_t two31 = int64_t(1) << 31;
-  const bool fits = 256 * (a.lda > a.ldb ? a.lda : a.ldb) * 2 + a.K * 2 < two31 &&
-                    256 * a.ldc * 4 < two31;
-  if (a.N % 256 == 0 && fits) {
-    // Fewer 256x256 tiles than CUs (a single document's forward, e.g. the
-    // 768-wide projections at a few thousand rows): the same kernel on 128x128
-    // tiles over 2x2 waves.  The wave tile keeps its 64 columns, the K order
-    // per output and the per-64-column norm partials, so every output is
-    // bit-identical to the 256x256 launch's.
-    const int64_t nb256 = ((a.M + 255) / 256) * (a.N / 256);
-    if (nb256 < device_cus()) return run_gemm_dma_epi<128, 128, 64, 2, 2>(a, s);
+  if (a.N % 256 == 0 && tile_reach_fits(a)) {
+    switch (pick_tile(a.M, a.N, a.K, a.epi == EPI_RESID_F32)) {
+      case T64x64: return run_gemm_pipe_epi<64, 64, 2, 1, 2, 5>(a, s);
+      case T64x128: return run_gemm_pipe_epi<64, 128, 2, 2, 4, 3>(a, s);
+      case T128x128: return run_gemm_pipe_epi<128, 128, 4, 2, 4, 5>(a, s);
+      case T128x256: return run_gemm_pipe_epi<128, 256, 2, 4, 4, 3>(a, s);
+      case T256x256: break;
+    }
+    if (a.row_ss) return fail(-2, "gemm: this launch does not take norm partials");
     return run_gemm_dma_epi<256, 256, 64, 2, 4>(a, s);
   }
+  if (a.row_ss) return fail(-2, "gemm: this launch does not take norm partials");
   return run_gemm<128, 128, 32, 2, 2, 2, 3>(a, s);
 }
 

@@ -1083,7 +1083,7 @@ __global__ __launch_bounds__(256) void row_rstd_kernel(const float* __restrict__
   const float* s = ss + r * np;
   float t = 0.f;
   for (int q = 0; q < np; ++q) t += s[q];
-  rstd[r] = 1.f / (sqrtf(t / (float)dim) + eps);
+  rstd[r] = row_factor(t, dim, eps);
 }
 
 int launch_row_rstd(const float* ss, float* rstd, int64_t rows, int np, int dim, float eps,

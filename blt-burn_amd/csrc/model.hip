@@ -277,7 +277,20 @@ int Model::forward(const int32_t* tokens, int64_t B, int64_t T, const blt_model_
                          carry ? ss : nullptr, carry ? attn_nw : nullptr)))
     return rc;
   const int np = (int)(D / 64);
-  if (carry && (rc = launch_row_rstd(ss, rstd, M, np, (int)D, cfg.norm_eps, s))) return rc;
+  // Small launches form the row factors from the norm partials themselves (a
+  // row_rstd launch is about 4.5 us of dependency latency, twice per layer);
+  // on full 256 x 256 tiles those scattered loads cost more than the launch.
+  const bool qkv_ss = carry && gemm_takes_norm_partials(M, 3 * D, D, np);
+  const bool w13_ss = carry && gemm_takes_norm_partials(M, 2 * F, D, np);
+  auto row_factors = [&](GemmArgs& g, bool from_ss) {
+    if (from_ss) {
+      g.row_ss = ss; g.row_np = np; g.row_dim = (int)D; g.row_eps = cfg.norm_eps;
+    } else {
+      g.row_scale = rstd;
+    }
+  };
+  if (carry && !qkv_ss && (rc = launch_row_rstd(ss, rstd, M, np, (int)D, cfg.norm_eps, s)))
+    return rc;
   if ((rc = mark(BLT_STAGE_EMBED, s))) return rc;
   for (int64_t l = 0; l < cfg.n_layers; ++l) {
     GemmArgs g{};
@@ -288,7 +301,7 @@ int Model::forward(const int32_t* tokens, int64_t B, int64_t T, const blt_model_
     // the attention kernel's scores then come out of the MFMA in the log2 domain
     g.q_cols = (int)D; g.q_scale = kAttnQScale;
     g.seg_start = seg_start;
-    g.row_scale = rstd;
+    row_factors(g, qkv_ss);
     if ((rc = launch_gemm(g, s))) return rc;
     if ((rc = mark(BLT_STAGE_QKV_GEMM, s))) return rc;
     AttnArgs at{};
@@ -306,12 +319,12 @@ int Model::forward(const int32_t* tokens, int64_t B, int64_t T, const blt_model_
     g.M = M; g.N = D; g.K = D; g.lda = D; g.ldb = D; g.ldc = D; g.epi = EPI_RESID_F32;
     g.xb_out = a; g.ss_out = ss; g.ss_np = np; g.col_scale = ffn_nw + l * D;
     if ((rc = launch_gemm(g, s))) return rc;
-    if ((rc = launch_row_rstd(ss, rstd, M, np, (int)D, cfg.norm_eps, s))) return rc;
+    if (!w13_ss && (rc = launch_row_rstd(ss, rstd, M, np, (int)D, cfg.norm_eps, s))) return rc;
     if ((rc = mark(BLT_STAGE_O_GEMM, s))) return rc;
     g = GemmArgs{};
     g.A = a; g.Bt = w13 + l * 2 * F * D; g.C = hbuf;
     g.M = M; g.N = 2 * F; g.K = D; g.lda = D; g.ldb = D; g.ldc = F; g.epi = EPI_SILU_GATE;
-    g.row_scale = rstd;
+    row_factors(g, w13_ss);
     if ((rc = launch_gemm(g, s))) return rc;
     if ((rc = mark(BLT_STAGE_W13_GEMM, s))) return rc;
     g = GemmArgs{};
@@ -322,7 +335,8 @@ int Model::forward(const int32_t* tokens, int64_t B, int64_t T, const blt_model_
       g.xb_out = a; g.ss_out = ss; g.ss_np = np; g.col_scale = attn_nw + (l + 1) * D;
     }
     if ((rc = launch_gemm(g, s))) return rc;
-    if (next && (rc = launch_row_rstd(ss, rstd, M, np, (int)D, cfg.norm_eps, s))) return rc;
+    if (next && !qkv_ss && (rc = launch_row_rstd(ss, rstd, M, np, (int)D, cfg.norm_eps, s)))
+      return rc;
     if ((rc = mark(BLT_STAGE_W2_GEMM, s))) return rc;
   }
   // Only what the caller asked for: the head (final norm, logits, entropy)

@@ -115,13 +115,21 @@ struct GemmArgs {
   // col_scale (optional, [N] f32) multiplies column c of that bf16 copy only
   // (the consumer's RMSNorm weight): xb_out = bf16(residual * col_scale).
   // Consumer: a GEMM with row_scale set (its A is such a scaled bf16 residual)
-  // multiplies output row r by row_scale[r] before its epilogue.
+  // multiplies output row r by row_scale[r] before its epilogue; or, with
+  // row_ss set instead (gemm_takes_norm_partials), by the factor it forms from
+  // the row's row_np norm partials, row_dim and row_eps.
   uint16_t* xb_out;
   float* ss_out;
   int ss_np;
   const float* row_scale;
   const float* col_scale;
+  const float* row_ss;  // [M, row_np] f32, 16-byte aligned
+  int row_np, row_dim;
+  float row_eps;
 };
+// whether a (non-residual) launch of this shape with np norm partials per row
+// forms the row factors itself (row_ss); otherwise it needs row_scale
+bool gemm_takes_norm_partials(int64_t M, int64_t N, int64_t K, int np);
 int launch_gemm(const GemmArgs& a, hipStream_t s);
 
 // k_attn.hip -----------------------------------------------------------------

@@ -270,6 +270,24 @@ def test_full_size_properties():
         assert int(ln[b, :c[b]].sum()) == T
 
 
+def test_prefixes_of_any_length_bit_exact():
+    # Launches of every size give a row's values bit for bit: the GEMMs change
+    # tile with the number of rows, and below a full chip form the RMSNorm row
+    # factors from the norm partials instead of reading row_rstd's.
+    cfg = M.entropy_model_config()
+    cfg.n_layers = 2
+    w = M.random_weights(cfg, 12, hidden=2048)
+    B, T = 8, 8192
+    tok = torch.from_numpy(synth.tokens(synth.config_seed(4) + 1, (B, T))).cuda()
+    m = M.LMTransformer(cfg, w, device=0, max_tokens=B * T, window=300)
+    out = m.forward_with_embeddings(tok)
+    for n in (1, 2, 33, 64, 65, 200, 1024, 1100, 1999, 2600, 4096, 6144, 7000):
+        pre = m.forward_with_embeddings(tok[3:4, :n].contiguous())
+        for name in ("logits", "pre_norm_embeddings", "embedding_norms", "entropies",
+                     "coherence_scores"):
+            assert torch.equal(getattr(pre, name)[0], getattr(out, name)[3, :n]), (n, name)
+
+
 def test_from_safetensors_matches_in_memory_weights(tmp_path):
     """A facebook/blt-entropy style checkpoint (PyTorch [out, in] layout) loads
     to the same model: outputs are bit-identical to the in-memory weights, and

@@ -611,6 +611,42 @@ def test_gemm_small_launch_tiles_bit_identical(epi, K):
     assert torch.equal(small, big[:Ms])
 
 
+# Every tile the launch selection picks between (64 x 64 up to 128 x 256, one
+# block per tile with loader waves) at the edges of its row tiles, with K tiles
+# fewer than, equal to and more than the stages: bit-identical to the same rows
+# of a 256 x 256 launch.
+@pytest.mark.parametrize("K", [64, 256, 320, 2048])
+@pytest.mark.parametrize("epi", ["bf16", "resid", "f32", "silu", "qkv"])
+def test_gemm_every_launch_tile_bit_identical(epi, K):
+    # eight full rounds of 256 x 256 tiles: always that tile
+    Mb = 256 * (130 if epi == "silu" else 230 if epi == "qkv" else 690)
+    N = {"silu": 4096, "qkv": 2304}.get(epi, 768)
+    torch.manual_seed(7)
+    a = torch.randn(Mb, K, device=DEV).to(torch.bfloat16)
+    bt = (0.05 * torch.randn(N, K, device=DEV)).to(torch.bfloat16)
+    kw = {}
+    if epi == "qkv":
+        kw = dict(rope_cols=1536, seq_len=512,
+                  cs=torch.from_numpy(oracle.rope_table(64, 512, 10000.0)).to(DEV))
+    if epi == "f32":
+        kw = dict(n_valid=N)
+    code = {"bf16": _lib.EPI_BF16, "resid": _lib.EPI_RESID_F32, "f32": _lib.EPI_F32,
+            "silu": _lib.EPI_SILU_GATE, "qkv": _lib.EPI_QKV_ROPE}[epi]
+    if epi in ("resid", "f32"):
+        base = torch.randn(Mb, N, device=DEV)
+    else:
+        base = torch.zeros(Mb, N // 2 if epi == "silu" else N, device=DEV, dtype=torch.bfloat16)
+    big = base.clone()
+    _gemm_epi(a, bt, big, code, **kw)
+    guard = 70  # rows past M stay as they are
+    for M in (1, 31, 33, 63, 65, 127, 129, 300, 513, 1000, 1500, 2100, 2561, 3100, 4200, 5121,
+              6150, 8200, 10300):
+        small = base[:M + guard].clone()
+        _gemm_epi(a[:M].contiguous(), bt, small[:M], code, **kw)
+        assert torch.equal(small[:M], big[:M]), M
+        assert torch.equal(small[M:], base[M:M + guard]), M
+
+
 # ---------------------------------------------------------------- measurement probes
 def test_probe_copy_and_mfma():
     L = _lib.lib()
