@@ -25,6 +25,8 @@
 // key j visible to query i iff j <= i), extended with a window W > 0
 // (also j > i - W).  Tiles entirely outside a wave's visible band are
 // skipped; fully visible tiles skip the per-element mask.
+#include <type_traits>
+
 #include "rowops.hpp"
 
 namespace blt {
@@ -436,102 +438,281 @@ int run_attention(const AttnArgs& a, hipStream_t s) {
   return 0;
 }
 
-// ---- exact f32 attention: the reference kernel's semantics -----------------
+// ---- f32 attention: the reference kernel's semantics ------------------------
 // fused_attention_kernel (attention_kernel.rs:20-125): any head_dim up to 256,
 // Tq and Tkv independent, causal means key j visible to query i iff j <= i,
-// scores (q . k) * (1 / sqrt(d)) and the softmax in f32 throughout.  One
-// block per (batch, head, 32 queries): the query tile, and 32-key tiles of K
-// and V, in LDS; thread t owns query t / 8 and, in the score step, keys
-// t % 8 + 8 m (m < 4), in the output step, head-dim columns t % 8 + 8 c; an
-// online softmax carries the running max and sum across key tiles.
-constexpr int FQ = 32, FK = 32, F_MAXD = 256;
+// scores (q . k) * (1 / sqrt(d)) and the softmax in f32 throughout.
+//
+// Both contractions run on the f32 matrix cores (v_mfma_f32_32x32x2_f32: f32
+// products and sums, 157 TFLOP/s), which is what bounds it: a 32-query x 32-key
+// step of d = 64 is 64 MFMAs of 64 cycles beside about 130 VALU instructions.
+// One block = 32 queries of one (batch, head); its four waves take every fourth
+// 32-key tile and meet once at the end, so a single document's few hundred
+// queries still give the chip 4 waves per 32 of them and no barrier sits in the
+// key loop.  As in attn_fwd_kernel the scores are S^T = K . Q^T (a lane owns one
+// query) and O^T += V^T . P^T with P^T straight from the score registers: the
+// lane of half h holds keys 8 (r / 4) + 4 h + r % 4 in register r, so PV step r
+// contracts the key pair {8 (r / 4) + r % 4, + 4} and V's operand is row 8 (r / 4)
+// + 4 h + r % 4.  QK^T contracts d in the order 8 j +
+// 4 h + e, one 16-byte piece of the lane's K row per four MFMAs.  Operands come
+// from global memory into registers (a tile's V under its QK^T MFMAs, the next
+// tile's K under its PV MFMAs); the waves of a block read neighbouring tiles, and
+// the blocks of one head share an XCD's L2.
+// Measured us, before (32-query blocks whose threads formed dot products from
+// LDS on the VALU) and now: B = 2, H = 12, T = 1000, d = 64, causal 994 -> 53;
+// B = 4, H = 12, T = 2048, d = 64, full 6720 -> 590 (87 TFLOP/s); B = 1, H = 4, T
+// = 2048, d = 128, causal 2310 -> 78.  Without its K and V loads the full case
+// takes 390 us: what is left is the loads, K's 32 rows x 32 bytes per
+// instruction above all.  The largest error against 64 bits is no larger than
+// the VALU kernel's (2.6e-7 against 3.3e-7 rel on the first case).
+constexpr int F_MAXD = 256;
 
+// ROW: how rows are read: 2 = d is 32 ND, 16-byte rows; 1 = d % 4 == 0, 16-byte
+// rows; 0 = element by element.
+template <int ND, int ROW>
 __global__ __launch_bounds__(256) void attn_f32_kernel(const float* __restrict__ q,
                                                        const float* __restrict__ k,
                                                        const float* __restrict__ v,
-                                                       float* __restrict__ o, int64_t H,
-                                                       int64_t Tq, int64_t Tkv, int d,
-                                                       int causal, float scale) {
-  extern __shared__ float smem[];
-  const int dp = d + 1;  // K row pitch: the 8 key rows a score step reads fall in distinct banks
-  float* Qs = smem;                // [FQ][d]
-  float* Ks = Qs + FQ * d;         // [FK][dp]
-  float* Vs = Ks + FK * dp;        // [FK][d]
-  float* Ps = Vs + FK * d;         // [FQ][FK + 1]
-  const int tid = threadIdx.x, qi = tid >> 3, g = tid & 7;
-  const int64_t q0 = (int64_t)blockIdx.x * FQ;
-  const int64_t bh = (int64_t)blockIdx.z * H + blockIdx.y;
+                                                       float* __restrict__ o, int64_t Tq,
+                                                       int64_t Tkv, int d, int causal,
+                                                       int hgroup, float cs) {
+  // e^(x / sqrt(d)), cs = log2(e) / sqrt(d)
+  auto expw = [&](float x) { return __builtin_amdgcn_exp2f(x * cs); };
+  constexpr int NW = 4, NC = 4 * ND;     // waves; 8-wide chunks of the head dim
+  constexpr int OP = 32 * ND + 4;        // output row pitch in LDS (floats)
+  // a whole V tile in registers beside K's, where that leaves two waves per SIMD
+  constexpr bool VPRE = ROW == 2 ? ND <= 4 : ND <= 2;
+  __shared__ __attribute__((aligned(16))) float so[NW * 32 * OP];
+  __shared__ float sm[NW][32], sl[NW][32];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l31 = lane & 31, h = lane >> 5;
+
+  // Dispatch places block i on XCD i % 8: each XCD takes a contiguous run of
+  // ids.  Ids walk groups of `hgroup` heads (whose K and V fit an XCD's L2),
+  // query blocks from the last (the longest causal rows) down, heads fastest,
+  // so the blocks a CU holds together have different lengths.
+  const int64_t nqb = gridDim.x, nbh = (int64_t)gridDim.y * gridDim.z, nb = nqb * nbh;
+  const int64_t bid = blockIdx.x + nqb * (blockIdx.y + (int64_t)gridDim.y * blockIdx.z);
+  const int64_t nb8 = nb & ~(int64_t)7;
+  const int64_t id = bid < nb8 ? (bid & 7) * (nb8 >> 3) + (bid >> 3) : bid;
+  const int64_t grp = id / (nqb * hgroup), rem = id - grp * nqb * hgroup;
+  const int64_t gh = nbh - grp * hgroup < hgroup ? nbh - grp * hgroup : hgroup;
+  const int64_t bh = grp * hgroup + rem % gh, q0 = (nqb - 1 - rem / gh) * 32;
   const float* qb = q + bh * Tq * d;
   const float* kb = k + bh * Tkv * d;
   const float* vb = v + bh * Tkv * d;
-  for (int i = tid; i < FQ * d; i += 256) {
-    const int r = i / d;
-    Qs[i] = q0 + r < Tq ? qb[(q0 + r) * d + (i % d)] : 0.f;
-  }
-  const int nd = (d + 7) / 8;  // output columns per thread
-  float acc[F_MAXD / 8];
+  const int nc = (d + 7) / 8;
+
+  // the lane's pieces of one row: elements 8 j + 4 h .. + 3, zero past d
+  auto load_row = [&](const float* row, f32x4_t (&f)[NC]) {
 #pragma unroll
-  for (int c = 0; c < F_MAXD / 8; ++c) acc[c] = 0.f;
-  float m = -INFINITY, l = 0.f;
-  const int64_t qabs = q0 + qi;
-  const int64_t kend = causal ? (q0 + FQ < Tkv ? q0 + FQ : Tkv) : Tkv;
-  for (int64_t k0 = 0; k0 < kend; k0 += FK) {
-    __syncthreads();  // the previous tile's K, V and P are no longer read
-    for (int i = tid; i < FK * d; i += 256) {
-      const int r = i / d, e = i % d;
-      const bool in = k0 + r < Tkv;
-      Ks[r * dp + e] = in ? kb[(k0 + r) * d + e] : 0.f;
-      Vs[i] = in ? vb[(k0 + r) * d + e] : 0.f;
-    }
-    __syncthreads();
-    float sc[4];
-    float mt = -INFINITY;
+    for (int j = 0; j < NC; ++j) {
+      const int c = 8 * j + 4 * h;
+      if constexpr (ROW == 2) {
+        f[j] = *reinterpret_cast<const f32x4_t*>(row + c);
+      } else if constexpr (ROW == 1) {
+        const f32x4_t x = *reinterpret_cast<const f32x4_t*>(row + (c < d ? c : 0));
+        f[j] = c < d ? x : f32x4_t{0.f, 0.f, 0.f, 0.f};
+      } else {
 #pragma unroll
-    for (int m2 = 0; m2 < 4; ++m2) {
-      const int kj = g + 8 * m2;
-      float dot = 0.f;
-      for (int e = 0; e < d; ++e) dot += Qs[qi * d + e] * Ks[kj * dp + e];
-      const int64_t kabs = k0 + kj;
-      const bool vis = kabs < Tkv && (!causal || kabs <= qabs);
-      sc[m2] = vis ? dot * scale : -INFINITY;
-      mt = fmaxf(mt, sc[m2]);
-    }
-    // the query's 32 scores of this tile sit in 8 consecutive lanes
-#pragma unroll
-    for (int x = 1; x < 8; x <<= 1) mt = fmaxf(mt, __shfl_xor(mt, x, 8));
-    const float m_new = fmaxf(m, mt);
-    const float alpha = m == -INFINITY ? (m_new == -INFINITY ? 1.f : 0.f) : expf(m - m_new);
-    float ls = 0.f;
-#pragma unroll
-    for (int m2 = 0; m2 < 4; ++m2) {
-      const float pv = m_new == -INFINITY ? 0.f : expf(sc[m2] - m_new);
-      Ps[qi * (FK + 1) + g + 8 * m2] = pv;
-      ls += pv;
-    }
-#pragma unroll
-    for (int x = 1; x < 8; x <<= 1) ls += __shfl_xor(ls, x, 8);
-    l = l * alpha + ls;
-    m = m_new;
-#pragma unroll
-    for (int c = 0; c < F_MAXD / 8; ++c) acc[c] *= alpha;
-    __syncthreads();  // P of the tile complete
-    for (int kj = 0; kj < FK; ++kj) {
-      const float pk = Ps[qi * (FK + 1) + kj];
-#pragma unroll
-      for (int c = 0; c < F_MAXD / 8; ++c) {
-        const int e = g + 8 * c;
-        if (c < nd && e < d) acc[c] += pk * Vs[kj * d + e];
+        for (int e = 0; e < 4; ++e) {
+          const float x = row[c + e < d ? c + e : 0];
+          f[j][e] = c + e < d ? x : 0.f;
+        }
       }
     }
-  }
-  if (qabs >= Tq) return;
-  const float inv = l > 0.f ? 1.f / l : 0.f;
-  float* orow = o + (bh * Tq + qabs) * d;
+  };
+  const int64_t qi = q0 + l31;
+  f32x4_t qf[NC], kf[NC];
+  load_row(qb + (qi < Tq ? qi : Tq - 1) * d, qf);
+
+  const int64_t kend = causal && q0 + 32 < Tkv ? q0 + 32 : Tkv;
+  const int64_t ntile = (kend + 31) / 32;
+  // row addresses are a uniform tile base and a 32-bit lane offset
+  const int dd = ROW == 2 ? 32 * ND : d;
+  auto load_k = [&](int64_t t) {
+    const int64_t left = Tkv - 1 - t * 32;  // the tile's last valid row
+    load_row(kb + t * 32 * dd + (unsigned)((l31 < left ? l31 : (int)left) * dd), kf);
+  };
+  // V is read in VW-wide pieces: row i of O^T block n is head-dim column VW i + n
+  // % VW + 32 VW (n / VW).  Columns past d: rows of O^T that are never stored.
+  constexpr int VW = ROW == 0 ? 1 : ND % 4 == 0 ? 4 : ND % 2 == 0 ? 2 : 1;
+  constexpr int NV = ND / VW;
+  typedef float vf_t __attribute__((ext_vector_type(VW)));
+  int dcol[NV];
 #pragma unroll
-  for (int c = 0; c < F_MAXD / 8; ++c) {
-    const int e = g + 8 * c;
-    if (c < nd && e < d) orow[e] = acc[c] * inv;
+  for (int n = 0; n < NV; ++n) {
+    const int c = VW * l31 + 32 * VW * n;
+    dcol[n] = ROW == 2 || c < d ? c : d - VW;
   }
+
+  f32x16_t oacc[ND];
+#pragma unroll
+  for (int n = 0; n < ND; ++n)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) oacc[n][r] = 0.f;
+  float m = -INFINITY, l = 0.f;  // l: this lane's half of the keys
+
+  // one 32-key tile; PART: its last keys are past Tkv
+  auto tile = [&](int64_t t, auto part) {
+    constexpr bool PART = decltype(part)::value;
+    const int64_t k0 = t * 32;
+    const float* vt = vb + k0 * dd;
+    const int last = PART ? (int)(Tkv - 1 - k0) : 31;  // the tile's last valid key
+    // V of key k0 + 8 (r / 4) + 4 h + r % 4; zero past Tkv
+    auto load_v = [&](int n, vf_t (&f)[16]) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int kr = 8 * (r >> 2) + (r & 3);
+        if constexpr (PART) {
+          const int key = kr + 4 * h;
+          const vf_t x = *reinterpret_cast<const vf_t*>(
+              vt + (unsigned)((key < last ? key : last) * dd + dcol[n]));
+#pragma unroll
+          for (int u = 0; u < VW; ++u) f[r][u] = key <= last ? x[u] : 0.f;
+        } else {
+          f[r] = *reinterpret_cast<const vf_t*>(
+              vt + ((unsigned)(4 * h * dd + dcol[n]) + (unsigned)(kr * dd)));
+        }
+      }
+    };
+    vf_t vf[VPRE ? NV : 1][16];
+    if constexpr (VPRE) {
+#pragma unroll
+      for (int n = 0; n < NV; ++n) load_v(n, vf[n]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    f32x16_t s;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) s[r] = 0.f;
+#pragma unroll
+    for (int j = 0; j < NC; ++j)
+      if (ROW == 2 || j < NC - 7 || j < nc) {  // chunks wholly past d hold zeros
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          s = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[j][e], qf[j][e], s, 0, 0, 0);
+      }
+    __builtin_amdgcn_sched_barrier(0);
+    // (unconditional, so the wait for V below leaves these loads in flight; after
+    // the wave's last tile they re-read one of its rows)
+    load_k(t + NW < ntile ? t + NW : t);
+    // mask: key > query (causal) or past Tkv
+    if (PART || (causal && k0 + 31 > q0)) {
+      const int64_t qrel = qi - k0;
+      const int lim = causal && qrel < last ? (int)qrel : last;  // last visible key
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s[r] = 8 * (r >> 2) + (r & 3) <= lim - 4 * h ? s[r] : -INFINITY;
+    }
+    float mt = s[0];
+#pragma unroll
+    for (int r = 1; r < 16; ++r) mt = fmaxf(mt, s[r]);
+    {
+      float a, b;
+      swap_pair<32>(mt, a, b);
+      mt = fmaxf(a, b);
+    }
+    // the scores are relative to the running max before the scale, so the
+    // exponent of every term that matters is small and nearly exact
+    const float m_new = fmaxf(m, mt);
+    const float mu = m_new == -INFINITY ? 0.f : m_new;
+    const float alpha = expw(m - mu);
+    m = m_new;
+    float ls = 0.f;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      s[r] = expw(s[r] - mu);
+      ls += s[r];
+    }
+    l = l * alpha + ls;
+#pragma unroll
+    for (int n = 0; n < ND; ++n)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) oacc[n][r] *= alpha;
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (VPRE) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+#pragma unroll
+        for (int n = 0; n < ND; ++n)
+          oacc[n] = __builtin_amdgcn_mfma_f32_32x32x2f32(vf[n / VW][r][n % VW], s[r], oacc[n], 0,
+                                                         0, 0);
+    } else {
+#pragma unroll
+      for (int n = 0; n < NV; ++n) {
+        load_v(n, vf[0]);
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+#pragma unroll
+          for (int u = 0; u < VW; ++u)
+            oacc[n * VW + u] = __builtin_amdgcn_mfma_f32_32x32x2f32(vf[0][r][u], s[r],
+                                                                    oacc[n * VW + u], 0, 0, 0);
+      }
+    }
+  };
+  if (w < ntile) load_k(w);
+  const int64_t nwhole = Tkv / 32 < ntile ? Tkv / 32 : ntile;  // at most one partial tile
+  int64_t t = w;
+  for (; t < nwhole; t += NW) tile(t, std::false_type{});
+  if (t < ntile) tile(t, std::true_type{});
+
+  // ---- the four waves' partial results ----
+  {
+    float a, b;
+    swap_pair<32>(l, a, b);
+    l = a + b;
+  }
+  if (h == 0) {
+    sm[w][l31] = m;
+    sl[w][l31] = l;
+  }
+  __syncthreads();
+  float mx = sm[0][l31];
+#pragma unroll
+  for (int i = 1; i < NW; ++i) mx = fmaxf(mx, sm[i][l31]);
+  const float mu = mx == -INFINITY ? 0.f : mx;
+  const float wt = expw(m - mu);
+  float lt = 0.f;
+#pragma unroll
+  for (int i = 0; i < NW; ++i) lt += sl[i][l31] * expw(sm[i][l31] - mu);
+  // a query that sees no key gets 0
+  const float f = lt > 0.f ? wt / lt : 0.f;
+  float* orow = so + (w * 32 + l31) * OP;
+#pragma unroll
+  for (int n = 0; n < NV; ++n)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      vf_t x;
+#pragma unroll
+      for (int u = 0; u < VW; ++u) x[u] = oacc[n * VW + u][r] * f;
+      *reinterpret_cast<vf_t*>(orow + VW * (8 * (r >> 2) + 4 * h + (r & 3)) + 32 * VW * n) = x;
+    }
+  __syncthreads();
+  // the block's rows are one contiguous run of the output
+  const int nq = (int)(Tq - q0 < 32 ? Tq - q0 : 32);
+  float* dst = o + (bh * Tq + q0) * d;
+  for (int i = tid; i < nq * d; i += 256) {
+    const int r = i / d, c = i - r * d;
+    const float* p = so + r * OP + c;
+    dst[i] = (p[0] + p[32 * OP]) + (p[64 * OP] + p[96 * OP]);
+  }
+}
+
+template <int ND>
+int run_attention_f32(const float* q, const float* k, const float* v, float* o, int64_t B,
+                      int64_t H, int64_t Tq, int64_t Tkv, int d, int causal, hipStream_t s) {
+  const dim3 grid((unsigned)((Tq + 31) / 32), (unsigned)H, (unsigned)B);
+  const float cs = (float)(1.44269504088896340736 / sqrt((double)d));
+  const bool vec = d % 4 == 0 && (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v) & 15) == 0;
+  // heads whose K and V share half an XCD's 4 MB L2, at most an eighth of them
+  const int64_t fit = (int64_t)(2 << 20) / (Tkv * d * 8 + 1), share = (B * H + 7) / 8;
+  const int hgroup = (int)(fit < 1 ? 1 : fit < share ? fit : share);
+  auto kern = !vec ? attn_f32_kernel<ND, 0>
+                   : d == 32 * ND ? attn_f32_kernel<ND, 2> : attn_f32_kernel<ND, 1>;
+  hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, q, k, v, o, Tq, Tkv, d, causal ? 1 : 0, hgroup,
+                     cs);
+  BLT_LAUNCH_CHECK("attn_f32_kernel");
+  return 0;
 }
 
 }  // namespace
@@ -540,19 +721,16 @@ int launch_attention_f32(const float* q, const float* k, const float* v, float* 
                          int64_t H, int64_t Tq, int64_t Tkv, int d, int causal, hipStream_t s) {
   if (B == 0 || H == 0 || Tq == 0) return 0;
   if (d < 1 || d > F_MAXD) return fail(-2, "attention_f32: head_dim must be 1 .. 256");
-  if (H > 65535 || B > 65535 || (Tq + FQ - 1) / FQ > 0x7fffffff)
+  if (H > 65535 || B > 65535 || (Tq + 31) / 32 > 0x7fffffff)
     return fail(-2, "attention_f32: grid too large");
-  const size_t lds = (size_t)(FQ * d + FK * (d + 1) + FK * d + FQ * (FK + 1)) * sizeof(float);
-  // beyond the default 64 KB of dynamic LDS the kernel's limit is raised (a
-  // host-side setting of the current device, set on every such launch)
-  if (lds > 64 * 1024)
-    BLT_HIP_CHECK(hipFuncSetAttribute((const void*)attn_f32_kernel,
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-  const dim3 grid((unsigned)((Tq + FQ - 1) / FQ), (unsigned)H, (unsigned)B);
-  hipLaunchKernelGGL(attn_f32_kernel, grid, dim3(256), lds, s, q, k, v, o, H, Tq, Tkv, d,
-                     causal ? 1 : 0, 1.0f / sqrtf((float)d));
-  BLT_LAUNCH_CHECK("attn_f32_kernel");
-  return 0;
+  switch ((d + 31) / 32) {
+    case 1: return run_attention_f32<1>(q, k, v, o, B, H, Tq, Tkv, d, causal, s);
+    case 2: return run_attention_f32<2>(q, k, v, o, B, H, Tq, Tkv, d, causal, s);
+    case 3: return run_attention_f32<3>(q, k, v, o, B, H, Tq, Tkv, d, causal, s);
+    case 4: return run_attention_f32<4>(q, k, v, o, B, H, Tq, Tkv, d, causal, s);
+    case 5: case 6: return run_attention_f32<6>(q, k, v, o, B, H, Tq, Tkv, d, causal, s);
+    default: return run_attention_f32<8>(q, k, v, o, B, H, Tq, Tkv, d, causal, s);
+  }
 }
 
 int launch_attention(const AttnArgs& a, hipStream_t s) {

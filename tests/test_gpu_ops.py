@@ -500,6 +500,42 @@ def test_attention_f32_reference_kernel(B, H, Tq, Tkv, d, causal):
                                atol=1e-4, rtol=0)
 
 
+@pytest.mark.parametrize("d", [1, 4, 31, 36, 64, 96, 129, 160, 192, 252, 256])
+def test_attention_f32_tile_edges(d):
+    # query blocks and key tiles of 32 at their edges, more and fewer tiles than
+    # the block's four waves, every row-read form (whole 32-column blocks, d %
+    # 4 == 0, any d, and rows that are not 16-byte aligned), no key at all.
+    # Bound: scores of N(0, 1) data stay below 8 sqrt(d) / sqrt(d) * 4 = 32, so
+    # their f32 rounding (2^-24 of that, a few times over d products) moves a
+    # weight by some 1e-5 relative and the output, an average of |v| <= 5, by
+    # less than 5e-5; measured 2e-6.
+    L = _lib.lib()
+    stream = torch.cuda.current_stream().cuda_stream
+    for Tq, Tkv, causal, shift in [(1, 1, 1, 0), (32, 31, 0, 0), (33, 32, 1, 0), (31, 33, 0, 1),
+                                   (65, 129, 1, 0), (100, 161, 0, 1), (200, 96, 1, 1)]:
+        q, k, v = (synth.normal_f32(i + d + Tq, (2, 3, n, d))
+                   for i, n in ((301, Tq), (302, Tkv), (303, Tkv)))
+        dev = []
+        for x in (q, k, v):
+            buf = torch.empty(x.size + shift, device=DEV)
+            buf[shift:] = torch.from_numpy(x.reshape(-1))
+            dev.append(buf[shift:])
+        guard = 64
+        o = torch.full((q.size + guard,), 7.0, device=DEV)
+        _lib.check(L.blt_fused_attention_f32(*[t.data_ptr() for t in dev], o.data_ptr(), 2, 3, Tq,
+                                             Tkv, d, causal, stream), "attention_f32")
+        torch.cuda.synchronize()
+        assert torch.all(o[q.size:] == 7.0)
+        ref = oracle.attention_kernel(q, k, v, bool(causal))
+        np.testing.assert_allclose(o[:q.size].cpu().numpy().reshape(ref.shape), ref, atol=5e-5,
+                                   rtol=0, err_msg=str((Tq, Tkv, causal, shift)))
+    o = torch.full((2 * 3 * 5 * d,), 7.0, device=DEV)
+    q = torch.ones_like(o)
+    _lib.check(L.blt_fused_attention_f32(q.data_ptr(), None, None, o.data_ptr(), 2, 3, 5, 0, d, 1,
+                                         stream), "attention_f32")
+    assert torch.all(o == 0.0)
+
+
 def test_attention_f32_rejects_wide_heads():
     q = cuda(synth.normal_f32(90, (1, 1, 8, 264)))
     with pytest.raises(_lib.BltError):
