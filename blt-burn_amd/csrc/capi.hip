@@ -343,7 +343,7 @@ int blt_patch_means(const float* entropies, const float* norms, const float* coh
   if (B == 0) return BLT_OK;
   if (!entropies || !norms || !starts || !count)
     return fail(BLT_ERR_INVALID, "patch_means: null entropies, norms, starts or count");
-  return launch_patch_means(entropies, norms, coherence, starts, count, B, T, nullptr, nullptr,
+  return launch_patch_means(entropies, norms, coherence, starts, count, B, T, nullptr, nullptr, 0,
                             mean_entropy, mean_prominence, mean_coherence, STREAM(stream));
 }
 

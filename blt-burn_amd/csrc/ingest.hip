@@ -396,8 +396,8 @@ int Ingest::long_pass(int64_t d, LongDoc& ld, const int64_t* doc_off, int32_t* s
   if (pm.any()) {
     BLT_HIP_CHECK(hipMemcpyAsync(l_N, ld.N.data(), (size_t)L * 4, hipMemcpyHostToDevice, up));
     BLT_HIP_CHECK(hipMemcpyAsync(l_C, ld.C.data(), (size_t)L * 4, hipMemcpyHostToDevice, up));
-    if ((rc = launch_patch_means(l_H, l_N, l_C, l_starts, l_count, 1, 0, l_off, l_len, l_pH, l_pN,
-                                 l_pC, up)))
+    if ((rc = launch_patch_means(l_H, l_N, l_C, l_starts, l_count, 1, 0, l_off, l_len, L, l_pH,
+                                 l_pN, l_pC, up)))
       return rc;
   }
   int32_t n = 0;
@@ -654,6 +654,7 @@ int Ingest::run(const int32_t* tokens, const int64_t* doc_off, int64_t n_docs, f
         s.h_dest[r * T + c] = -1;
       }
     const int64_t nd = (int64_t)s.units.size();
+    const int64_t longest = nd > 0 ? *std::max_element(s.h_dlen, s.h_dlen + nd) : 0;
     stats.batches += 1;
     stats.row_tokens += BT;
     // ---- upload ----
@@ -682,7 +683,7 @@ int Ingest::run(const int32_t* tokens, const int64_t* doc_off, int64_t n_docs, f
       return rc;
     // per-patch means (pipeline.rs:240-258) over the same per-document rows
     if (pm.any() && (rc = launch_patch_means(s.d_H, s.d_N, s.d_C, s.d_starts, s.d_counts, nd, 0,
-                                             s.d_doff, s.d_dlen, s.d_pH, s.d_pN, s.d_pC, ks)))
+                                             s.d_doff, s.d_dlen, longest, s.d_pH, s.d_pN, s.d_pC, ks)))
       return rc;
     // pieces of arena documents: stitched on the device; the batch holding a
     // document's last piece runs its boundary pass and per-patch means
@@ -709,7 +710,7 @@ int Ingest::run(const int32_t* tokens, const int64_t* doc_off, int64_t n_docs, f
         return rc;
       if (pm.any() &&
           (rc = launch_patch_means(la_H, la_N, la_C, la_starts, la_count + ld.slot, 1, 0,
-                                   la_off + ld.slot, la_len + ld.slot, la_pH, la_pN, la_pC, ks)))
+                                   la_off + ld.slot, la_len + ld.slot, ld.L, la_pH, la_pN, la_pC, ks)))
         return rc;
       s.long_done.push_back(u.doc);
     }

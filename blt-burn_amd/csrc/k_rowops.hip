@@ -705,58 +705,72 @@ __global__ __launch_bounds__(PB_THREADS) void patch_boundary_kernel(
 // starts (ascending, as the boundary pass writes them) and the outputs share
 // the row offsets.
 //
-// One block per row walks it in tiles of PM_TILE positions staged in LDS with
-// coalesced loads.  Each patch that starts in a tile is one thread's serial
-// chain over the tile's LDS copy; the one patch that runs past the tile end
-// hands its partial sums (two LDS slots, alternating by tile) to thread 0 of
-// the next tile, which continues the same chain, so a patch of any length
-// costs LDS reads, not one dependent global load per element.
+// A row is cut into tiles of PM_TILE positions; a tile's block stages them in LDS
+// with coalesced loads, finds the first patch that starts there (a block-wide
+// search over the starts: 256 probes a round) and gives each (patch, signal)
+// pair of the patches that start in the tile one lane's serial chain.  The one
+// patch that runs past the tile end is the block's too: one wave goes on with its
+// chains, a signal per lane, while the other waves stage the next positions.
+// What bounds it is latency: the dependent loads of the search, and 4 cycles per
+// element of the longest chain.  [16, 8192], patches of 8 on average: 27 us with
+// one block per row walking its tiles, 8 us now; one row of 8,000 that is a single
+// patch: 70 us with one lane adding both signals in turn, 31 us now.
 // ---------------------------------------------------------------------------
 constexpr int PM_THREADS = 256;
-constexpr int PM_TILE = 2048;
+constexpr int PM_TILE = 1024;
 
-// One chain's sums over LDS positions [a, z), left to right: the reads go 16
-// bytes at a time and run ahead of the dependent adds (unrolled body), the
-// order of the adds is the element order.
-template <bool HAS_C>
-__device__ inline void pm_chain(const float* sH, const float* sN, const float* sC, int a, int z,
-                                float& sh, float& sn, float& sc) {
+// s plus x[a .. z), left to right (the order of the adds is the element order):
+// 16-byte reads, and in long spans the next 32 elements are read under the
+// dependent adds of the current 32 (scheduling barriers keep those reads ahead
+// of the adds, where the compiler would sink them behind).
+__device__ inline float pm_chain(const float* x, int a, int z, float s) {
   int t = a;
-  for (; t < z && (t & 3); ++t) {
-    sh += sH[t];
-    sn += sN[t];
-    if (HAS_C) sc += sC[t];
+  for (; t < z && (t & 3); ++t) s += x[t];
+  if (t + 96 <= z) {
+    float4 u[8], v[8];
+    auto load = [&](float4 (&d)[8], int at) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) d[i] = *reinterpret_cast<const float4*>(x + at + 4 * i);
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    auto add = [&](const float4 (&d)[8]) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        s += d[i].x; s += d[i].y; s += d[i].z; s += d[i].w;
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    load(u, t);
+    for (; t + 96 <= z; t += 64) {
+      load(v, t + 32);
+      add(u);
+      load(u, t + 64);
+      add(v);
+    }
+    add(u);
+    t += 32;
   }
 #pragma unroll 4
   for (; t + 4 <= z; t += 4) {
-    const float4 h = *reinterpret_cast<const float4*>(sH + t);
-    const float4 q = *reinterpret_cast<const float4*>(sN + t);
-    sh += h.x; sh += h.y; sh += h.z; sh += h.w;
-    sn += q.x; sn += q.y; sn += q.z; sn += q.w;
-    if (HAS_C) {
-      const float4 c = *reinterpret_cast<const float4*>(sC + t);
-      sc += c.x; sc += c.y; sc += c.z; sc += c.w;
-    }
+    const float4 h = *reinterpret_cast<const float4*>(x + t);
+    s += h.x; s += h.y; s += h.z; s += h.w;
   }
-  for (; t < z; ++t) {
-    sh += sH[t];
-    sn += sN[t];
-    if (HAS_C) sc += sC[t];
-  }
+  for (; t < z; ++t) s += x[t];
+  return s;
 }
 
-template <bool HAS_C>
+// NA signals: H, N and (NA = 3) C.  Block (b, y) of the grid takes the tiles y, y
+// + gridDim.y, ... of row b.
+template <int NA>
 __global__ __launch_bounds__(PM_THREADS) void patch_means_kernel(
     const float* __restrict__ H, const float* __restrict__ N, const float* __restrict__ C,
     const int32_t* __restrict__ starts, const int32_t* __restrict__ count, int64_t T_dense,
-    const int64_t* __restrict__ row_off, const int32_t* __restrict__ row_len,
-    float* __restrict__ mH, float* __restrict__ mN, float* __restrict__ mC,
-    const int64_t* __restrict__ out_off) {
-  __shared__ __attribute__((aligned(16))) float sH[PM_TILE];
-  __shared__ __attribute__((aligned(16))) float sN[PM_TILE];
-  __shared__ __attribute__((aligned(16))) float sC[HAS_C ? PM_TILE : 4];
-  __shared__ float carry[2][3];  // partial sums handed to the next tile
-  __shared__ int32_t last[2];    // last patch started in the tile (atomicMax)
+    const int64_t* __restrict__ row_off, const int32_t* __restrict__ row_len, float* mH, float* mN,
+    float* mC, const int64_t* __restrict__ out_off) {
+  __shared__ __attribute__((aligned(16))) float sx[2][NA][PM_TILE + 4];  // (+ 4: signals on other banks)
+  __shared__ float run_s[NA];   // sums of the patch that runs past the tile end
+  __shared__ int64_t run_st, run_e, run_p;
+  __shared__ int probes[PM_THREADS / 64];
   const int64_t b = blockIdx.x;
   const int64_t roff = row_off ? row_off[b] : b * T_dense;
   const int64_t T = row_len ? (int64_t)row_len[b] : T_dense;
@@ -764,7 +778,14 @@ __global__ __launch_bounds__(PM_THREADS) void patch_means_kernel(
   // without starts every row is one patch [0, T)
   int64_t n = starts ? (int64_t)count[b] : 1;
   n = n < 0 ? 0 : (n > T ? T : n);
-  const int tid = threadIdx.x;
+  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  auto in = [&](int a) { return a == 0 ? H : a == 1 ? N : C; };
+  // positions [u0, u0 + w) of every signal into buffer k, by threads t0, t0 + nt, ..
+  auto stage = [&](int k, int64_t u0, int w, int t0, int nt) {
+#pragma unroll
+    for (int a = 0; a < NA; ++a)
+      for (int i = t0; i < w; i += nt) sx[k][a][i] = in(a)[roff + u0 + i];
+  };
   // patch p's span, clamped to 0 <= st <= e <= T
   auto span = [&](int64_t p, int64_t& st, int64_t& e) {
     e = p + 1 < n ? (int64_t)starts[roff + p + 1] : T;
@@ -772,70 +793,80 @@ __global__ __launch_bounds__(PM_THREADS) void patch_means_kernel(
     st = starts ? (int64_t)starts[roff + p] : 0;
     st = st < 0 ? 0 : (st > e ? e : st);
   };
-  auto put = [&](int64_t p, float sh, float sn, float sc, int64_t len) {
-    const bool any = len > 0;
-    const float fl = (float)len;
-    if (mH) mH[ooff + p] = any ? sh / fl : 0.f;
-    if (mN) mN[ooff + p] = any ? sn / fl : 0.f;
-    if (mC) mC[ooff + p] = any ? sc / fl : 0.f;
+  auto put = [&](int a, int64_t p, float sum, int64_t len) {
+    float* m = a == 0 ? mH : a == 1 ? mN : mC;
+    if (m) m[ooff + p] = len > 0 ? sum / (float)len : 0.f;
   };
-  if (tid == 0) last[0] = -1;
-  int64_t p0 = 0;   // first patch that has not started in an earlier tile
-  int64_t cp = -1;  // patch continuing from the previous tile (-1: none)
-  int k = 0;
-  for (int64_t t0 = 0; t0 < T && (p0 < n || cp >= 0); t0 += PM_TILE, ++k) {
+  for (int64_t t0 = (int64_t)blockIdx.y * PM_TILE; t0 < T; t0 += (int64_t)gridDim.y * PM_TILE) {
     const int64_t t1 = t0 + PM_TILE < T ? t0 + PM_TILE : T;
-    const int w = (int)(t1 - t0);
-    for (int i = tid; i < w; i += PM_THREADS) {
-      sH[i] = H[roff + t0 + i];
-      sN[i] = N[roff + t0 + i];
-      if (HAS_C) sC[i] = C[roff + t0 + i];
-    }
-    __syncthreads();
-    // the next tile's counter, free since that tile's last read two syncs ago
-    if (tid == 0) last[(k + 1) & 1] = -1;
-    const int nc0 = cp >= 0 ? 1 : 0;  // chain 0 continues patch cp
-    for (int64_t j = tid;; j += PM_THREADS) {
-      int64_t p, st, e;
-      float sh = 0.f, sn = 0.f, sc = 0.f;
-      if (j < nc0) {
-        p = cp;
-        span(p, st, e);
-        sh = carry[k & 1][0];
-        sn = carry[k & 1][1];
-        sc = carry[k & 1][2];
+    const bool last_tile = t1 == T;
+    stage(0, t0, (int)(t1 - t0), tid, PM_THREADS);
+    if (tid == 0) run_e = 0;
+    // the first patch with starts[p] >= t0: lo .. hi brackets it, 256 probes
+    // split the bracket (starts ascend, so the passing probes are a prefix)
+    int64_t lo = 0, hi = t0 > 0 ? n : 0;
+    while (lo < hi) {
+      const int64_t step = (hi - lo + PM_THREADS - 1) / PM_THREADS;
+      const int64_t p = lo + tid * step;
+      const bool below = p < hi && (starts ? starts[roff + p] : 0) < t0;
+      const uint64_t bal = __ballot(below);
+      if (lane == 0) probes[wid] = __popcll(bal);
+      __syncthreads();
+      const int c = probes[0] + probes[1] + probes[2] + probes[3];
+      __syncthreads();
+      if (c == 0) {
+        hi = lo;
       } else {
-        p = p0 + (j - nc0);
-        if (p >= n) break;
-        span(p, st, e);
-        if (st >= t1) break;  // starts ascend: this and later patches start further on
-        atomicMax(&last[k & 1], (int32_t)p);
-      }
-      const int a = (int)((st > t0 ? st : t0) - t0);
-      const int z = (int)((e < t1 ? e : t1) - t0);
-      pm_chain<HAS_C>(sH, sN, sC, a, z, sh, sn, sc);
-      if (e <= t1) {
-        put(p, sh, sn, sc, e - st);
-      } else {  // only the tile's last chain runs on
-        carry[(k + 1) & 1][0] = sh;
-        carry[(k + 1) & 1][1] = sn;
-        carry[(k + 1) & 1][2] = sc;
+        const int64_t nlo = lo + (c - 1) * step + 1, nhi = lo + c * step;
+        lo = nlo;
+        hi = nhi < hi ? nhi : hi;
       }
     }
     __syncthreads();
-    // block-uniform: the patches that started here and the chain that runs on
-    const int64_t lp = last[k & 1];
-    const int64_t lastchain = lp >= p0 ? lp : cp;
-    if (lp >= p0) p0 = lp + 1;
-    cp = -1;
-    if (lastchain >= 0) {
+    for (int64_t j = tid;; j += PM_THREADS) {
+      const int64_t p = lo + j / NA;
+      const int a = (int)(j % NA);
+      if (p >= n) break;
       int64_t st, e;
-      span(lastchain, st, e);
-      if (e > t1) cp = lastchain;
+      span(p, st, e);
+      if (!last_tile && st >= t1) break;  // starts ascend: this and later ones lie further on
+      // (st < t0 only for starts that do not ascend)
+      const int x0 = (int)((st < t0 ? t0 : st > t1 ? t1 : st) - t0);
+      const int x1 = (int)((e < t1 ? (e < t0 ? t0 : e) : t1) - t0);
+      const float sum = pm_chain(sx[0][a], x0, x1, 0.f);
+      if (e <= t1) {
+        put(a, p, sum, e - st);
+      } else {  // only the tile's last patch runs on
+        run_s[a] = sum;
+        if (a == 0) {
+          run_st = st;
+          run_p = p;
+          run_e = e;
+        }
+      }
     }
+    __syncthreads();
+    const int64_t e = run_e;
+    if (e > t1) {
+      const int64_t st = run_st, p = run_p;
+      float sum = wid == 0 && lane < NA ? run_s[lane] : 0.f;
+      int k = 1;
+      stage(k, t1, (int)(e - t1 < PM_TILE ? e - t1 : PM_TILE), tid, PM_THREADS);
+      __syncthreads();
+      for (int64_t u0 = t1; u0 < e; u0 += PM_TILE, k ^= 1) {
+        const int64_t u1 = u0 + PM_TILE;
+        const int w = (int)(e - u0 < PM_TILE ? e - u0 : PM_TILE);
+        if (wid == 0) {
+          if (lane < NA) sum = pm_chain(sx[k][lane], 0, w, sum);
+        } else if (u1 < e) {
+          stage(k ^ 1, u1, (int)(e - u1 < PM_TILE ? e - u1 : PM_TILE), tid - 64, PM_THREADS - 64);
+        }
+        __syncthreads();
+      }
+      if (wid == 0 && lane < NA) put(lane, p, sum, e - st);
+    }
+    __syncthreads();  // the buffers and run_* are reused by the block's next tile
   }
-  // patches that start at or past the row end (only for malformed starts)
-  for (int64_t p = p0 + tid; p < n; p += PM_THREADS) put(p, 0.f, 0.f, 0.f, 0);
 }
 
 // ---------------------------------------------------------------------------
@@ -1210,15 +1241,29 @@ int launch_patch_boundaries_varlen(const float* H, const int64_t* row_off, const
 
 int launch_patch_means(const float* H, const float* N, const float* C, const int32_t* starts,
                        const int32_t* count, int64_t B, int64_t T, const int64_t* row_off,
-                       const int32_t* row_len, float* mH, float* mN, float* mC, hipStream_t s,
-                       const int64_t* out_off) {
+                       const int32_t* row_len, int64_t max_len, float* mH, float* mN, float* mC,
+                       hipStream_t s, const int64_t* out_off) {
   if (B == 0) return 0;
+  // one block per tile; a row without starts is one chain, so one block.  A
+  // caller's mean that overlaps an input keeps one block per row: it has read a
+  // position before it writes a mean there (patch p starts at p or later).
+  int64_t tiles = starts ? ((row_len ? max_len : T) + PM_TILE - 1) / PM_TILE : 1;
+  if (!row_len) {
+    auto overlap = [&](const float* m, const float* x) {
+      return m && x && m < x + B * T && x < m + B * T;
+    };
+    for (const float* m : {mH, mN, mC})
+      for (const float* x : {H, N, C})
+        if (overlap(m, x)) tiles = 1;
+  }
+  tiles = tiles < 1 ? 1 : tiles > 65535 ? 65535 : tiles;
+  const dim3 grid((unsigned)B, (unsigned)tiles);
   if (C)
-    hipLaunchKernelGGL(patch_means_kernel<true>, dim3((unsigned)B), dim3(PM_THREADS), 0, s, H, N,
-                       C, starts, count, T, row_off, row_len, mH, mN, mC, out_off);
+    hipLaunchKernelGGL(patch_means_kernel<3>, grid, dim3(PM_THREADS), 0, s, H, N, C, starts, count,
+                       T, row_off, row_len, mH, mN, mC, out_off);
   else
-    hipLaunchKernelGGL(patch_means_kernel<false>, dim3((unsigned)B), dim3(PM_THREADS), 0, s, H, N,
-                       C, starts, count, T, row_off, row_len, mH, mN, mC, out_off);
+    hipLaunchKernelGGL(patch_means_kernel<2>, grid, dim3(PM_THREADS), 0, s, H, N, C, starts, count,
+                       T, row_off, row_len, mH, mN, mC, out_off);
   BLT_LAUNCH_CHECK("patch_means_kernel");
   return 0;
 }

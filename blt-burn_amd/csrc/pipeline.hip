@@ -152,7 +152,7 @@ int Pipeline::suffix_pass(const float* H, const float* N, int64_t n) {
                                     v_count.as<int32_t>(), s)))
     return rc;
   if ((rc = launch_patch_means(H, N, nullptr, v_starts.as<int32_t>(), v_count.as<int32_t>(), 1, n,
-                               nullptr, nullptr, v_mH.as<float>(), v_mN.as<float>(), nullptr, s)))
+                               nullptr, nullptr, 0, v_mH.as<float>(), v_mN.as<float>(), nullptr, s)))
     return rc;
   BLT_HIP_CHECK(hipMemcpyAsync(hv_count.p, v_count.p, 4, hipMemcpyDeviceToHost, s));
   BLT_HIP_CHECK(hipMemcpyAsync(hv_starts.p, v_starts.p, b, hipMemcpyDeviceToHost, s));
@@ -367,7 +367,7 @@ int Pipeline::process_documents(const uint8_t* bytes, const int64_t* doc_off, in
     BLT_HIP_CHECK(hipMemcpyAsync(v_lens.p, hv_starts.p, nc * 4, hipMemcpyHostToDevice, s));
     const int64_t* d_off = v_off.as<int64_t>();
     if ((r = launch_patch_means(v_H.as<float>(), v_N.as<float>(), nullptr, nullptr, nullptr,
-                                (int64_t)nc, 0, d_off, v_lens.as<int32_t>(), v_mH.as<float>(),
+                                (int64_t)nc, 0, d_off, v_lens.as<int32_t>(), 0, v_mH.as<float>(),
                                 v_mN.as<float>(), nullptr, s, d_off + nc)))
       return r;
     BLT_HIP_CHECK(hipMemcpyAsync(hv_mH.p, v_mH.p, nc * 4, hipMemcpyDeviceToHost, s));

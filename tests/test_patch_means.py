@@ -136,6 +136,39 @@ def test_device_long_patches_bit_exact(T):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("T", [1, 1023, 1024, 1025, 2049, 70000])
+def test_device_means_at_tile_edges_bit_exact(T):
+    """One block per 1024-position tile: patches that start and end on tile
+    edges, patches over several tiles (with and without starts inside the tiles
+    they cross), more starts than one search round of 256 probes resolves, and
+    means written over the inputs they come from."""
+    import torch
+    from blt_burn_amd import patcher
+    rng = np.random.default_rng(T)
+    edges = [t for e in range(1024, T, 1024) for t in (e - 1, e, e + 1) if t < T]
+    rows = [[0], list(range(T)), [0] + [t for t in edges if t > 0], [0] + list(range(1024, T, 1024)),
+            [0] + [t for t in (5, 1500, 3000, 69000) if t < T],
+            [0] + sorted(rng.choice(np.arange(1, T), T // 8, replace=False).tolist()) if T > 8
+            else [0]]
+    rows = [sorted(set(r)) for r in rows]
+    B = len(rows)
+    H = rng.normal(3.0, 1.0, (B, T)).astype(np.float32)
+    N = (rng.random((B, T)) * 30).astype(np.float32)
+    st, ct = _starts(rows, T)
+    rH, rN, rC = oracle.patch_means(H, N, st, ct, H)
+    Hd, Nd, sd, cd = (torch.from_numpy(x).cuda() for x in (H, N, st, ct))
+    for C, out in ((None, None), (Hd, None), (None, (Hd.clone(), Nd.clone(), None))):
+        h, n = (out[0], out[1]) if out else (Hd, Nd)  # out: in place
+        mH, mN, mC = patcher.patch_means(h, n, sd, cd, C, out=out)
+        for b in range(B):
+            k = ct[b]
+            assert np.array_equal(mH.cpu().numpy()[b, :k], rH[b, :k]), (T, b)
+            assert np.array_equal(mN.cpu().numpy()[b, :k], rN[b, :k]), (T, b)
+            if C is not None:
+                assert np.array_equal(mC.cpu().numpy()[b, :k], rC[b, :k]), (T, b)
+
+
+@pytest.mark.gpu
 def test_device_rejects_bad_out_tensors():
     import torch
     from blt_burn_amd import BltError, patcher
