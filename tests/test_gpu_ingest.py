@@ -215,6 +215,33 @@ def test_ingest_config5_vs_oracle_entropy_model():
           "embeddings max rel=%.2e" % (lens, *worst))
 
 
+@pytest.mark.parametrize("lens", [[1], [64], [120], [121], [128], [60, 60], [100, 128, 5],
+                                  [113, 112, 111, 110], [128] * 4, [30] * 9])
+def test_ingest_partial_batches(lens):
+    """A batch runs only its used rows, cut to the longest fill when a
+    sixteenth of the row is free (rows of 128: up to 120 tokens): every
+    document's outputs, embeddings included, are its own forward's.  Not bit for
+    bit: the attention's running max moves for a whole wave of 32 queries at
+    once, so the padding queries beside a document's last ones can shift its
+    rounding of the bf16 softmax numerators (2^-9 each).  The bounds are the
+    other packed-row tests'; a wrong row, stride or position moves the outputs by
+    their own size."""
+    cfg = M.LMTransformerConfig(**TINY)
+    w = M.random_weights(cfg, 27, hidden=256)
+    m = M.LMTransformer(cfg, w, device=0, max_tokens=4 * 128, window=0)
+    ing = I.StreamingIngest(m, I.BltConfig(threshold=0.3, max_seq_len=128, chunk_overlap=0),
+                            rows=4, row_len=128, with_embeddings=True)
+    toks, off = _docs(synth.config_seed(5) + 21, lens)
+    res = ing.run(toks, off)
+    for d in range(len(lens)):
+        t = torch.from_numpy(toks[off[d]:off[d + 1]][None].astype(np.int32)).cuda()
+        o = m.forward_with_embeddings(t)
+        _check_doc_outputs(res, d, o.entropies.cpu().numpy()[0],
+                           o.embedding_norms.cpu().numpy()[0], 5e-3, 5e-3, 0.3, 0)
+        E, ref = res.doc(d)[5], o.pre_norm_embeddings.cpu().numpy()[0]
+        assert np.abs(E - ref).max() <= 1e-2 * np.abs(ref).max()
+
+
 def test_process_bytes_mirror():
     cfg = M.LMTransformerConfig(**TINY)
     w = M.random_weights(cfg, 25, hidden=256)
