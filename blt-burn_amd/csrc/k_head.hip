@@ -74,10 +74,14 @@ __device__ inline void head_split(const f32x4_t (&xv)[8], const float* wrow, flo
     ss = fmaf(x4.w, x4.w, ss);
     const f32x4_t a = x4 * w4;
     const uint32_t h01 = pack_bf16x2(a.x, a.y), h23 = pack_bf16x2(a.z, a.w);
-    const uint32_t l01 = pack_bf16x2(a.x - __builtin_bit_cast(float, h01 << 16),
-                                     a.y - __builtin_bit_cast(float, h01 & 0xffff0000u));
-    const uint32_t l23 = pack_bf16x2(a.z - __builtin_bit_cast(float, h23 << 16),
-                                     a.w - __builtin_bit_cast(float, h23 & 0xffff0000u));
+    // the remainder from the unrounded product, so that every kernel that
+    // splits gets the same bits whatever the compiler contracts
+    const uint32_t l01 =
+        pack_bf16x2(fmaf(x4.x, w4.x, -__builtin_bit_cast(float, h01 << 16)),
+                    fmaf(x4.y, w4.y, -__builtin_bit_cast(float, h01 & 0xffff0000u)));
+    const uint32_t l23 =
+        pack_bf16x2(fmaf(x4.z, w4.z, -__builtin_bit_cast(float, h23 << 16)),
+                    fmaf(x4.w, w4.w, -__builtin_bit_cast(float, h23 & 0xffff0000u)));
     // elements 4 i .. 4 i + 3 of the lane's 32 = step i / 2, slots 4 (i % 2) ..
     u32x4_t* ph = reinterpret_cast<u32x4_t*>(&ahi[i >> 1]);
     u32x4_t* pl = reinterpret_cast<u32x4_t*>(&alo[i >> 1]);
@@ -85,6 +89,42 @@ __device__ inline void head_split(const f32x4_t (&xv)[8], const float* wrow, flo
     (*ph)[2 * (i & 1) + 1] = h23;
     (*pl)[2 * (i & 1)] = l01;
     (*pl)[2 * (i & 1) + 1] = l23;
+  }
+}
+
+// The row's entropy, norm and coherence from its finished logits: lane l holds
+// row l % 32's columns of half h in block order, mx their maximum (-inf past V);
+// lanes l and l ^ 32 share the row.  H = log sum p - sum(p d) / sum p with d = x
+// - max, p = e^d: the same quantity as -sum exp(lsm) lsm (patcher.rs:38-63).
+__device__ inline void head_finish(const f32x16_t (&acc)[HD_NB], float mx, float nrm, int64_t row,
+                                   int h, bool in, float* ent, float* norms, float* coh) {
+  {
+    float a, b;
+    swap_pair<32>(mx, a, b);
+    mx = fmaxf(a, b);
+  }
+  float sp = 0.f, sd = 0.f;
+#pragma unroll
+  for (int j = 0; j < HD_NB; ++j)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const float d = fmaxf(acc[j][r] - mx, -1e30f);
+      const float pe = __expf(d);
+      sp += pe;
+      sd = fmaf(pe, d, sd);
+    }
+  {
+    float a, b;
+    swap_pair<32>(sp, a, b);
+    sp = a + b;
+    swap_pair<32>(sd, a, b);
+    sd = a + b;
+  }
+  if (h == 0 && in) {
+    const float H = __logf(sp) - sd * __builtin_amdgcn_rcpf(sp);
+    if (ent) ent[row] = H;
+    if (norms) norms[row] = nrm;
+    if (coh) coh[row] = nrm * nrm / (H + 1e-6f);
   }
 }
 
@@ -265,35 +305,166 @@ void head_entropy_kernel(const float* __restrict__ x, const float* __restrict__ 
       wave_lds_fence_head();
     }
   }
-  {
-    float a, b;
-    swap_pair<32>(mx, a, b);
-    mx = fmaxf(a, b);
+  head_finish(acc, mx, nrm, row, h, row < M, ent, norms, coh);
+}
+
+// Launches of few rows: 32 rows per block, so that a document of a few hundred
+// tokens uses more than a couple of CUs, and a quarter of the nine column blocks
+// per wave (3, 2, 2, 2), so that the serial walk over K is 24 MFMAs per K tile
+// instead of 72.  What bounds it is that walk's latency.  Each K tile's weights
+// (36 KB) and x rows (8 KB, 16-byte pieces XOR-swizzled by row) move by LDS DMA
+// through three stages, two tiles in flight; every wave splits the x tile for
+// itself.  The finished logits meet in LDS, where one wave forms the entropies
+// in head_entropy_kernel's order per lane while the others store the logits:
+// every output is bit-identical to that kernel's.
+// M = 48: 36 -> 19 us; M = 8192 (256 blocks): 38 -> 22 us; from the second round of
+// blocks on the wide kernel is ahead (M = 12288: 38 against 40 us).
+constexpr int HS_STAGES = 3;
+constexpr int HS_ROWS = 32;
+constexpr int HS_XTILE = HS_ROWS * HD_BK * 4;         // bytes of x per K tile
+constexpr int HS_STAGE = HD_TILE + HS_XTILE;
+constexpr int HS_QW = HD_CHUNKS / HD_WAVES;           // weight chunks per wave
+constexpr int HS_QX = HS_XTILE / 1024 / HD_WAVES;     // x chunks per wave
+constexpr int HS_Q = HS_QW + HS_QX;
+constexpr int HS_LP = HD_NPAD + 4;                    // logits pitch in LDS (floats)
+constexpr int64_t kHeadSmallRows = 8192;
+static_assert(HS_ROWS * HS_LP * 4 <= HS_STAGES * HS_STAGE, "staged logits fit the stages");
+
+template <bool LOGITS>
+__global__ __launch_bounds__(256)
+void head_entropy_small_kernel(const float* __restrict__ x, const float* __restrict__ wn,
+                               const uint16_t* __restrict__ wt, int64_t M, int D, int V, float eps,
+                               float* __restrict__ logits, float* __restrict__ ent,
+                               float* __restrict__ norms, float* __restrict__ coh) {
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[HS_STAGES * HS_STAGE];
+  __shared__ __attribute__((aligned(16))) float wn_s[HD_DMAX];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lrow = lane & 31, h = lane >> 5;
+  const int64_t row0 = (int64_t)blockIdx.x * HS_ROWS;
+  const int64_t row = row0 + lrow;
+  const int KT = D / HD_BK;
+  const unsigned lds_base = (unsigned)(uintptr_t)lds;
+  // this wave's column blocks: 0, 1, 2; 3, 4; 5, 6; 7, 8 (the others' third
+  // accumulator repeats a block and is dropped: no branch in the K loop)
+  const int j0 = wid == 0 ? 0 : 1 + 2 * wid, nb = wid == 0 ? 3 : 2;
+  auto block = [&](int j) { return j0 + j < HD_NB ? j0 + j : HD_NB - 1; };
+
+  // x chunk (q, wid) holds rows 4 (4 q + wid) .. + 3: slot s of row r takes the
+  // 16-byte piece s ^ (r % 16); rows past M read the last row, store nothing
+  const int last = (int)(M - 1 - row0 < HS_ROWS - 1 ? M - 1 - row0 : HS_ROWS - 1);
+  unsigned xoff[HS_QX];
+#pragma unroll
+  for (int q = 0; q < HS_QX; ++q) {
+    const int r = 4 * (4 * q + wid) + (lane >> 4);
+    xoff[q] = (unsigned)((r < last ? r : last) * D * 4 + (((lane & 15) ^ (r & 15)) << 4));
   }
-  // H = log sum p - sum(p d) / sum p with d = x - max, p = e^d: the same
-  // quantity as -sum exp(lsm) lsm (patcher.rs:38-63)
-  float sp = 0.f, sd = 0.f;
+  const float* xbase = x + row0 * D;
+  auto dma_tile = [&](int kt, int st) {
+    const unsigned char* src = reinterpret_cast<const unsigned char*>(wt) + (int64_t)kt * HD_TILE;
+    const unsigned sb = lds_base + (unsigned)(st * HS_STAGE);
 #pragma unroll
-  for (int j = 0; j < HD_NB; ++j)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const float d = fmaxf(acc[j][r] - mx, -1e30f);
-      const float pe = __expf(d);
-      sp += pe;
-      sd = fmaf(pe, d, sd);
+    for (int q = 0; q < HS_QW; ++q) {
+      const unsigned c = (unsigned)(q * HD_WAVES + wid) * 1024u;
+      dma16_so(src + c, (unsigned)lane * 16u, sb + c);
     }
+#pragma unroll
+    for (int q = 0; q < HS_QX; ++q)
+      dma16_so(xbase + kt * HD_BK, xoff[q],
+               sb + (unsigned)(HD_TILE + (q * HD_WAVES + wid) * 1024));
+  };
+
+  for (int i = tid * 4; i < D; i += 256 * 4)
+    *reinterpret_cast<f32x4_t*>(wn_s + i) = *reinterpret_cast<const f32x4_t*>(wn + i);
+  __syncthreads();  // (before the DMA: its counter is the loads' too)
+#pragma unroll
+  for (int t = 0; t < HS_STAGES - 1; ++t)
+    if (t < KT) dma_tile(t, t);
+
+  f32x16_t acc[3];
+#pragma unroll
+  for (int j = 0; j < 3; ++j)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[j][r] = 0.f;
+  float ss = 0.f;
+  int st = 0, stn = HS_STAGES - 1;
+  for (int kt = 0; kt < KT; ++kt) {
+    // tile kt has landed (tile kt + 1 may be in flight), and every wave is past
+    // tile kt - 1, whose stage takes tile kt + 2
+    if (kt + 1 < KT) dma_wait_barrier<HS_Q>();
+    else dma_wait_barrier<0>();
+    if (kt + HS_STAGES - 1 < KT) dma_tile(kt + HS_STAGES - 1, stn);
+    const uint16_t* tile = reinterpret_cast<const uint16_t*>(lds + st * HS_STAGE);
+    const float* xrow = reinterpret_cast<const float*>(lds + st * HS_STAGE + HD_TILE) + lrow * HD_BK;
+    f32x4_t xv[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      xv[i] = *reinterpret_cast<const f32x4_t*>(xrow + (((8 * h + i) ^ (lrow & 15)) << 2));
+    bf16x8_t ahi[4], alo[4];
+    float sst = 0.f;
+    head_split<0, 8>(xv, wn_s + kt * HD_BK + 32 * h, sst, ahi, alo);
+    ss = kt == 0 ? sst : ss + sst;
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      bf16x8_t wf[3];
+#pragma unroll
+      for (int j = 0; j < 3; ++j)
+        wf[j] =
+            *reinterpret_cast<const bf16x8_t*>(tile + head_swz(32 * block(j) + lrow, 4 * h + ks));
+#pragma unroll
+      for (int j = 0; j < 3; ++j)
+        acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[j], ahi[ks], acc[j], 0, 0, 0);
+#pragma unroll
+      for (int j = 0; j < 3; ++j)
+        acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[j], alo[ks], acc[j], 0, 0, 0);
+    }
+    stn = st;
+    st = st + 1 < HS_STAGES ? st + 1 : 0;
+  }
+
   {
     float a, b;
-    swap_pair<32>(sp, a, b);
-    sp = a + b;
-    swap_pair<32>(sd, a, b);
-    sd = a + b;
+    swap_pair<32>(ss, a, b);
+    ss = a + b;
   }
-  if (h == 0 && row < M) {
-    const float H = __logf(sp) - sd * __builtin_amdgcn_rcpf(sp);
-    if (ent) ent[row] = H;
-    if (norms) norms[row] = nrm;
-    if (coh) coh[row] = nrm * nrm / (H + 1e-6f);
+  const float nrm = sqrtf(ss);
+  const float rs = 1.f / (sqrtf(ss / (float)D) + eps);
+  __syncthreads();  // every wave is past its last read of the stages
+  float* lg = reinterpret_cast<float*>(lds);
+#pragma unroll
+  for (int j = 0; j < 3; ++j)
+    if (j < 2 || nb == 3) {
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        *reinterpret_cast<f32x4_t*>(lg + lrow * HS_LP + 32 * (j0 + j) + 8 * g + 4 * h) =
+            f32x4_t{acc[j][4 * g] * rs, acc[j][4 * g + 1] * rs, acc[j][4 * g + 2] * rs,
+                    acc[j][4 * g + 3] * rs};
+    }
+  __syncthreads();
+  if (wid == 0) {
+    f32x16_t v[HD_NB];
+    float mx = -INFINITY;
+#pragma unroll
+    for (int j = 0; j < HD_NB; ++j)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const int col = 32 * j + 8 * g + 4 * h;
+        const f32x4_t q = *reinterpret_cast<const f32x4_t*>(lg + lrow * HS_LP + col);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          v[j][4 * g + e] = col + e < V ? q[e] : -INFINITY;
+          mx = fmaxf(mx, v[j][4 * g + e]);
+        }
+      }
+    head_finish(v, mx, nrm, row, h, row < M, ent, norms, coh);
+  } else if (LOGITS) {
+    // the block's rows are one contiguous run of the output
+    const int v4 = V / 4, n4 = (last + 1) * v4;
+    f32x4_t* dst = reinterpret_cast<f32x4_t*>(logits + row0 * V);
+    for (int q = tid - 64; q < n4; q += 192) {
+      const int r = q / v4, c = q - r * v4;
+      dst[q] = *reinterpret_cast<const f32x4_t*>(lg + r * HS_LP + 4 * c);
+    }
   }
 }
 
@@ -323,13 +494,11 @@ int launch_head_entropy(const float* x, const float* w_norm, const uint16_t* wpa
                                                        "D % 64 == 0, D <= 1024");
   if (((uintptr_t)x | (uintptr_t)w_norm | (uintptr_t)logits) % 16)
     return fail(BLT_ERR_SHAPE, "head: 16-byte aligned residual, norm weight and logits");
-  const unsigned grid = ceil_div(M, HD_ROWS);
-  if (logits)
-    hipLaunchKernelGGL(head_entropy_kernel<true>, dim3(grid), dim3(256), 0, s, x, w_norm, wpacked,
-                       M, D, V, eps, logits, ent, norms, coh);
-  else
-    hipLaunchKernelGGL(head_entropy_kernel<false>, dim3(grid), dim3(256), 0, s, x, w_norm,
-                       wpacked, M, D, V, eps, logits, ent, norms, coh);
+  const bool small = M <= kHeadSmallRows;
+  auto kern = small ? (logits ? head_entropy_small_kernel<true> : head_entropy_small_kernel<false>)
+                    : (logits ? head_entropy_kernel<true> : head_entropy_kernel<false>);
+  hipLaunchKernelGGL(kern, dim3(ceil_div(M, small ? HS_ROWS : HD_ROWS)), dim3(256), 0, s, x, w_norm,
+                     wpacked, M, D, V, eps, logits, ent, norms, coh);
   BLT_LAUNCH_CHECK("head_entropy_kernel");
   return 0;
 }

@@ -288,6 +288,42 @@ def test_prefixes_of_any_length_bit_exact():
             assert torch.equal(getattr(pre, name)[0], getattr(out, name)[3, :n]), (n, name)
 
 
+@pytest.mark.parametrize("vocab,dim", [(260, 768), (4, 128), (100, 64), (256, 256), (288, 1024)])
+def test_head_launch_forms_bit_identical(vocab, dim):
+    # a model without layers is embedding + head.  Rows of the 32-row-block head
+    # (up to 8192 rows; at the edges of its blocks and of their last, partial one)
+    # equal the same rows of the 128-row-block head, for every output and with
+    # the logits left out.
+    cfg = M.LMTransformerConfig(dim=dim, n_layers=0, n_heads=dim // 64, max_seqlen=8192,
+                                vocab_size=vocab)
+    # norm weights and embeddings of more than 8 mantissa bits between them, so
+    # that the head's hi + lo split of their f32 product is exercised
+    w = M.random_weights(cfg, 15, hidden=128, std=0.5, norm_std=0.3)
+    big = torch.from_numpy(synth.tokens(synth.config_seed(4) + 15, (2, 4200)) % vocab).cuda()
+    m = M.LMTransformer(cfg, w, device=0, max_tokens=8400, hidden=128)
+    ref = m.forward_with_embeddings(big)  # 8400 rows: 128-row blocks
+    assert torch.isfinite(ref.entropies).all()
+    for n in (1, 2, 31, 32, 33, 63, 65, 100, 1000, 4097):
+        out = m.forward_with_embeddings(big[:1, :n].contiguous())
+        for name in ("logits", "embedding_norms", "entropies", "coherence_scores"):
+            assert torch.equal(getattr(out, name)[0], getattr(ref, name)[0, :n]), (n, name)
+    o = _lib_outputs(m, big[:1, :33].contiguous())
+    assert torch.equal(o, ref.entropies[0, :33])
+
+
+def _lib_outputs(m, tok):
+    """Entropies alone (no logits) through the C ABI."""
+    import ctypes
+    from blt_burn_amd import _lib
+    H = torch.empty(tok.shape[1], device="cuda")
+    o = _lib.ModelOutputs(None, None, None, H.data_ptr(), None)
+    _lib.check(_lib.lib().blt_model_forward(m._h, tok.data_ptr(), 1, tok.shape[1],
+                                            ctypes.byref(o),
+                                            torch.cuda.current_stream().cuda_stream), "forward")
+    torch.cuda.synchronize()
+    return H
+
+
 def test_from_safetensors_matches_in_memory_weights(tmp_path):
     """A facebook/blt-entropy style checkpoint (PyTorch [out, in] layout) loads
     to the same model: outputs are bit-identical to the in-memory weights, and
