@@ -831,6 +831,63 @@ void gemm_bf16_dma_persistent_kernel(GemmArgs p) {
   }
 }
 
+// The residual epilogue of a 64-column tile whose waves hold 32 x 32 pieces of it
+// (TM = TN = 1): the pieces meet in LDS, and wave w of the NW then finishes rows w
+// BM / NW .. of the tile with epilogue_lds's arithmetic and lane layout (16 lanes
+// of 4 columns per row).  rin holds the residual pieces of those rows.
+template <int BM, int NW>
+struct ResidRows {
+  static constexpr int RW = BM / NW;       // rows per wave
+  static constexpr int NP = RW * 16 / 64;  // 16-byte pieces per lane
+  f32x4_t res[NP];
+  f32x4_t csc;
+  __device__ inline void load(const GemmArgs& p, int64_t m0, int64_t n0, int wid, int lane) {
+#pragma unroll
+    for (int t = 0; t < NP; ++t) {
+      const int64_t row = m0 + wid * RW + (lane + 64 * t) / 16;
+      res[t] = *reinterpret_cast<const f32x4_t*>(reinterpret_cast<const float*>(p.C) +
+                                                 (row < p.M ? row : p.M - 1) * p.ldc + n0 +
+                                                 (lane & 15) * 4);
+    }
+    csc = f32x4_t{1.f, 1.f, 1.f, 1.f};
+    if (p.col_scale) csc = *reinterpret_cast<const f32x4_t*>(p.col_scale + n0 + (lane & 15) * 4);
+  }
+  __device__ inline void finish(const GemmArgs& p, const f32x16_t& acc, float rs, int64_t m0,
+                                int64_t n0, int wid, int wm, int wn, int lane, float* buf) {
+    constexpr int LD = 64 + 2;  // f32 row pitch (8-byte pad)
+    {
+      float* d = buf + (wm * 32 + (lane & 31)) * LD + wn * 32 + 4 * (lane >> 5);
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) d[8 * g + e] = acc[4 * g + e] * rs;
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+#pragma unroll
+    for (int t = 0; t < NP; ++t) {
+      const int r = wid * RW + (lane + 64 * t) / 16, c = (lane & 15) * 4;
+      const float* sp = buf + r * LD + c;
+      const f32x4_t v = f32x4_t{sp[0], sp[1], sp[2], sp[3]} + res[t];
+      const int64_t row = m0 + r;
+      const bool ok = row < p.M;
+      float ss = 0.f;
+      if (ok) {
+        *reinterpret_cast<f32x4_t*>(reinterpret_cast<float*>(p.C) + row * p.ldc + n0 + c) = v;
+        if (p.xb_out) {
+          const f32x4_t y = v * csc;
+          *reinterpret_cast<u32x2_t*>(p.xb_out + row * p.ldc + n0 + c) =
+              u32x2_t{pack_bf16x2(y.x, y.y), pack_bf16x2(y.z, y.w)};
+          ss = v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w;
+        }
+      }
+      if (p.ss_out) {
+        ss = sum16(ss);
+        if ((lane & 15) == 0 && ok) p.ss_out[row * p.ss_np + n0 / 64] = ss;
+      }
+    }
+  }
+};
+
 // The row factors of a consumer that forms them itself: the norm partials of
 // this lane's rows (p.row_np of them, a multiple of 4 up to 16) are loaded
 // before the K loop, and finish() sums them after it in row_rstd_kernel's
@@ -877,9 +934,9 @@ struct RowNorms {
 // alone 44 ns per K tile, the DMA issue 81 ns, fragment reads and MFMAs 170 ns,
 // and in one set of waves these add (11.8 us; deeper stages, the DMA spread
 // over the K steps and fragment reads ahead of the barrier changed nothing).
-// With the DMA in waves of its own the launch takes 9.6 us, against 24 us for
-// the two-stage persistent kernel on 128 x 128 tiles, whose every K tile waits
-// for the one load in flight.  For the same reason the epilogue's global inputs
+// With the DMA in waves of its own the launch takes 9.6 us (8.6 with the tile's
+// MFMAs on four waves, ResidRows), against 24 us for the two-stage persistent
+// kernel on 128 x 128 tiles, whose every K tile waits for the one load in flight.  For the same reason the epilogue's global inputs
 // (row factors or norm partials, the residual, the RoPE pairs) are requested
 // before the K loop.
 //
@@ -902,6 +959,8 @@ __global__ __launch_bounds__(64 * (WM * WN + NL)) void gemm_bf16_pipe_kernel(Gem
   constexpr int SLAB = C::TM > 1 ? 2 : 1;
   static_assert(NW * 32 * SLAB * (C::WTN + 4) * 2 <= S * SB && NW * 32 * (C::WTN + 2) * 4 <= S * SB,
                 "staged epilogue must fit in the stages");
+  constexpr bool PIECES = C::WTN == 32;  // waves of 32 x 32 pieces: the residual epilogue only
+  static_assert(!PIECES || (EPI == EPI_RESID_F32 && C::WTM == 32 && BN == 64), "see ResidRows");
   __shared__ __attribute__((aligned(1024))) unsigned char lds[S * SB];
 
   const int tid = threadIdx.x, lane = tid & 63;
@@ -977,8 +1036,10 @@ __global__ __launch_bounds__(64 * (WM * WN + NL)) void gemm_bf16_pipe_kernel(Gem
   f32x4_t cs0[8];
   const bool rope = EPI == EPI_QKV_ROPE && col0 < p.rope_cols;
   if (PRE && rope) load_rope_cs(p, row0 + lrow, lane, cs0);
+  ResidRows<BM, NW> rows;
+  if constexpr (PIECES) rows.load(p, m0, n0, wid, lane);
   ResidIn<C> rin;
-  if (PRE && EPI == EPI_RESID_F32 && row0 < p.M && col0 < p.N) {
+  if (!PIECES && PRE && EPI == EPI_RESID_F32 && row0 < p.M && col0 < p.N) {
     const int mrem = (int)(p.M - row0 < C::WTM ? p.M - row0 : C::WTM);
     const int nrem = (int)(p.N - col0 < C::WTN ? p.N - col0 : C::WTN);
     rin.load_slab(reinterpret_cast<const char*>(reinterpret_cast<const float*>(p.C) +
@@ -1029,7 +1090,10 @@ __global__ __launch_bounds__(64 * (WM * WN + NL)) void gemm_bf16_pipe_kernel(Gem
   if (!PRE && rope) load_rope_cs(p, row0 + lrow, lane, cs0);
   if (p.row_ss) rn.finish(p, rs);
   lds_barrier();
-  epilogue_lds<C, EPI, PRE, false>(p, acc, m0, n0, wid, wm, wn, lane, lds, rs, cs0, rin);
+  if constexpr (PIECES)
+    rows.finish(p, acc[0][0], rs[0], m0, n0, wid, wm, wn, lane, reinterpret_cast<float*>(lds));
+  else
+    epilogue_lds<C, EPI, PRE, false>(p, acc, m0, n0, wid, wm, wn, lane, lds, rs, cs0, rin);
 }
 
 }  // namespace gemm

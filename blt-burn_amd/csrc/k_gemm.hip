@@ -62,7 +62,13 @@ int run_gemm_pipe_epi(GemmArgs a, hipStream_t s) {
   switch (a.epi) {
     case EPI_BF16: return run_gemm_pipe<BM, BN, WM, WN, NL, S, EPI_BF16>(a, s);
     case EPI_F32: return run_gemm_pipe<BM, BN, WM, WN, NL, S, EPI_F32>(a, s);
-    case EPI_RESID_F32: return run_gemm_pipe<BM, BN, WM, WN, NL, S, EPI_RESID_F32>(a, s);
+    case EPI_RESID_F32:
+      // four waves of 32 x 32 pieces instead of two of 32 x 64: half the MFMA
+      // chain per K tile (M = 48, K = 2048: 9.9 -> 8.6 us; K = 768: 6.2 -> 5.5)
+      if constexpr (BM == 64 && BN == 64)
+        return run_gemm_pipe<64, 64, 2, 2, 4, S, EPI_RESID_F32>(a, s);
+      else
+        return run_gemm_pipe<BM, BN, WM, WN, NL, S, EPI_RESID_F32>(a, s);
     case EPI_QKV_ROPE: return run_gemm_pipe<BM, BN, WM, WN, NL, S, EPI_QKV_ROPE>(a, s);
     case EPI_SILU_GATE: return run_gemm_pipe<BM, BN, WM, WN, NL, S, EPI_SILU_GATE>(a, s);
   }
@@ -76,25 +82,27 @@ int run_gemm_pipe_epi(GemmArgs a, hipStream_t s) {
 // e per tile for the epilogue of its class (residual, other), the last term the
 // memory traffic that grows with the whole launch (r: the residual's).  The
 // constants are least-squares fits to the measured times of the four projection
-// shapes of the model (N, K = 2304, 768; 768, 768; 4096, 768; 768, 2048) at M = 48
-// .. 40000; over those 72 launches the tile it picks is within 8 % of the best of
-// eleven tried (mean 0.8 %).  Measured us (256 x 256 | picked), N = 768, K =
-// 2048: M = 48: 45.5 | 9.6 (64 x 64); 1536: 49.8 | 13.1 (64 x 128); 4096: 50.1 |
-// 20.1 (128 x 128); 8192: 52.4 | 32.4 (128 x 256); 40000: 143 | 143 (128 x 256: 154).
-// All tiles give bit-identical results, so the choice is free of M.
+// shapes of the model (N, K = 2304, 768; 768, 768; 4096, 768; 768, 2048) at M = 16
+// .. 40000; over those launches the tile it picks is within 7 % of the best
+// (mean 0.4 %).  Measured us (256 x 256 | picked), N = 768, K = 2048: M = 48: 46.7 |
+// 8.6 (64 x 64); 2048: 52.5 | 14.7 (64 x 128); 4096: 50.1 | 20.1 (128 x 128); 8192:
+// 52.4 | 32.4 (128 x 256); 40000: 143 | 143 (128 x 256: 154).  All tiles give
+// bit-identical results, so the choice is free of M.
 enum Tile { T64x64, T64x128, T128x128, T128x256, T256x256 };
 struct TileCost {
   int bm, bn;
   double fix, k, e_resid, e_other, kf, r;
 };
 constexpr TileCost kTileCost[] = {
-    {64, 64, 4.393, 0.164, 0.036, 0.422, 0.011, 0.841},
-    {64, 128, 3.267, 0.269, 0.075, 0.626, 0.004, 1.774},
-    {128, 128, 1.160, 0.341, 2.711, 3.454, 0.078, 4.828},
-    {128, 256, 1.039, 0.533, 5.597, 5.132, 0.212, 5.656},
-    {256, 256, 2.580, 1.167, 6.264, 6.274, 0.308, 11.024},
+    {64, 64, 3.263, 0.151, 0.358, 0.716, 0.008, 0.837},
+    {64, 128, 3.124, 0.264, 0.642, 0.425, 0.024, 1.067},
+    {128, 128, 1.030, 0.341, 3.705, 3.510, 0.071, 3.861},
+    {128, 256, 0.182, 0.558, 6.278, 6.044, 0.120, 6.608},
+    {256, 256, 2.072, 1.178, 8.411, 6.376, 0.304, 7.037},
 };
-Tile pick_tile(int64_t M, int64_t N, int64_t K, bool resid) {
+// a consumer of norm partials on 256 x 256 tiles needs the row_rstd launch
+constexpr double kRowFactorLaunch = 4.5;
+Tile pick_tile(int64_t M, int64_t N, int64_t K, bool resid, bool norm) {
   const int cus = device_cus() > 0 ? device_cus() : 256;
   const double KT = (double)(K / 64);
   const int64_t nb256 = ((M + 255) / 256) * (N / 256);
@@ -107,6 +115,7 @@ Tile pick_tile(int64_t M, int64_t N, int64_t K, bool resid) {
     const double c = (double)((n + cus - 1) / cus), f = (double)n / cus;
     double est = w.fix + c * (w.k * KT + (resid ? w.e_resid : w.e_other)) +
                  f * (w.kf * KT + (resid ? w.r : 0.0));
+    if (i == T256x256 && norm) est += kRowFactorLaunch;
     // a full chip of 256 x 256 tiles moves the fewest operand bytes: leave it
     // only for a clear gain
     if (i == T256x256 && nb256 >= cus) est *= 0.95;
@@ -139,7 +148,7 @@ int run_gemm(const GemmArgs& a, hipStream_t s) {
 // (dense operands: the model's launches)
 bool gemm_takes_norm_partials(int64_t M, int64_t N, int64_t K, int np) {
   return np % 4 == 0 && np <= 16 && N % 256 == 0 && K * 512 + K * 2 < (int64_t(1) << 31) &&
-         N * 1024 < (int64_t(1) << 31) && pick_tile(M, N, K, false) != T256x256;
+         N * 1024 < (int64_t(1) << 31) && pick_tile(M, N, K, false, true) != T256x256;
 }
 
 int launch_gemm(const GemmArgs& a_in, hipStream_t s) {
@@ -171,7 +180,7 @@ int launch_gemm(const GemmArgs& a_in, hipStream_t s) {
   // tile pick_tile chooses.  Otherwise (the 260-wide head, huge strides)
   // 128x128 register-staged tiles over 4 waves.
   if (a.N % 256 == 0 && tile_reach_fits(a)) {
-    switch (pick_tile(a.M, a.N, a.K, a.epi == EPI_RESID_F32)) {
+    switch (pick_tile(a.M, a.N, a.K, a.epi == EPI_RESID_F32, a.row_ss != nullptr)) {
       case T64x64: return run_gemm_pipe_epi<64, 64, 2, 1, 2, 5>(a, s);
       case T64x128: return run_gemm_pipe_epi<64, 128, 2, 2, 4, 3>(a, s);
       case T128x128: return run_gemm_pipe_epi<128, 128, 4, 2, 4, 5>(a, s);
