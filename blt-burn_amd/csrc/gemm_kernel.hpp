@@ -934,11 +934,12 @@ struct RowNorms {
 // alone 44 ns per K tile, the DMA issue 81 ns, fragment reads and MFMAs 170 ns,
 // and in one set of waves these add (11.8 us; deeper stages, the DMA spread
 // over the K steps and fragment reads ahead of the barrier changed nothing).
-// With the DMA in waves of its own the launch takes 9.6 us (8.6 with the tile's
-// MFMAs on four waves, ResidRows), against 24 us for the two-stage persistent
-// kernel on 128 x 128 tiles, whose every K tile waits for the one load in flight.  For the same reason the epilogue's global inputs
-// (row factors or norm partials, the residual, the RoPE pairs) are requested
-// before the K loop.
+// With the DMA in waves of its own the launch takes 9.6 us, with the tile's MFMAs
+// on four waves 8.6 (ResidRows), with fragment reads that cross the K tiles 8.2,
+// against 24 us for a two-stage persistent kernel on 128 x 128 tiles, whose every
+// K tile waits for the one load in flight.  For the same reason the epilogue's
+// global inputs (row factors or norm partials, the residual, the RoPE pairs) are
+// requested before the K loop.
 //
 // The wave tile keeps its 64 columns, the K order per output (from the last
 // tile down where the first column has bit 10 set) and the per-64-column norm
@@ -959,6 +960,14 @@ __global__ __launch_bounds__(64 * (WM * WN + NL)) void gemm_bf16_pipe_kernel(Gem
   constexpr int SLAB = C::TM > 1 ? 2 : 1;
   static_assert(NW * 32 * SLAB * (C::WTN + 4) * 2 <= S * SB && NW * 32 * (C::WTN + 2) * 4 <= S * SB,
                 "staged epilogue must fit in the stages");
+  // How far fragment reads run ahead of the MFMAs, and whether past the K tile's
+  // end.  128-row tiles: one step, across (N = 768, K = 2048, M = 6144 on 128 x
+  // 256: 30.0 -> 27.9 us; two or three steps cost them registers for nothing).
+  // 64 x 64, whose one wave per SIMD has nothing else to hide the LDS latency
+  // behind: three (M = 48: 8.6 -> 8.2 us).  64 x 128: not across, since two such
+  // blocks per CU already cover each other (W1|W3 at M = 1024: 10.8, across 10.9).
+  constexpr int AHEAD = BN == 64 ? 3 : 1;
+  constexpr bool CROSS = !(BM == 64 && BN == 128);
   constexpr bool PIECES = C::WTN == 32;  // waves of 32 x 32 pieces: the residual epilogue only
   static_assert(!PIECES || (EPI == EPI_RESID_F32 && C::WTM == 32 && BN == 64), "see ResidRows");
   __shared__ __attribute__((aligned(1024))) unsigned char lds[S * SB];
@@ -1067,26 +1076,45 @@ __global__ __launch_bounds__(64 * (WM * WN + NL)) void gemm_bf16_pipe_kernel(Gem
   };
   // this wave's LDS reads are done, and after the barrier every wave's are
   auto lds_barrier = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
-  bf16x8_t af[2][C::TM], bfr[2][C::TN];
+  // Fragments are read AHEAD K steps before their MFMAs, one set per step of the
+  // K tile; with CROSS the last steps of a tile read the first ones of the next,
+  // whose barrier they join with their own tile's MFMAs still to do.
+  constexpr int NK = BK / 16;
+  bf16x8_t af[NK][C::TM], bfr[NK][C::TN];
   int st = 0;  // stage of K tile t
-  for (int t = 0; t < KT; ++t) {
-    lds_barrier();
-    // fragments of K step ks + 1 are read beside the MFMAs of step ks
-    load_frags(st, 0, af[0], bfr[0]);
-    static_for<0, BK / 16>([&](auto kc) {
-      constexpr int ks = decltype(kc)::value;
-      if constexpr (ks + 1 < BK / 16) load_frags(st, ks + 1, af[(ks + 1) & 1], bfr[(ks + 1) & 1]);
+  auto k_tile = [&](auto last) {
+    const int next = st + 1 < S ? st + 1 : 0;
+    if constexpr (!CROSS) {
+      lds_barrier();
+      load_frags(st, 0, af[0], bfr[0]);
+    }
+    static_for<0, NK>([&](auto kc) {
+      constexpr int ks = decltype(kc)::value, kr = (ks + AHEAD) % NK;
+      if constexpr (ks + AHEAD < NK) {
+        load_frags(st, kr, af[kr], bfr[kr]);
+      } else if constexpr (CROSS && !decltype(last)::value) {
+        if constexpr (kr == 0) lds_barrier();
+        load_frags(next, kr, af[kr], bfr[kr]);
+      }
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int i = 0; i < C::TM; ++i)
 #pragma unroll
         for (int j = 0; j < C::TN; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bfr[ks & 1][j], af[ks & 1][i],
-                                                              acc[i][j], 0, 0, 0);
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bfr[ks][j], af[ks][i], acc[i][j], 0,
+                                                              0, 0);
       __builtin_amdgcn_sched_barrier(0);
     });
-    st = st + 1 < S ? st + 1 : 0;
+    st = next;
+  };
+  if constexpr (CROSS) {
+    lds_barrier();
+    static_for<0, AHEAD>([&](auto kc) {
+      load_frags(0, decltype(kc)::value, af[decltype(kc)::value], bfr[decltype(kc)::value]);
+    });
   }
+  for (int t = 0; t + 1 < KT; ++t) k_tile(std::false_type{});
+  k_tile(std::true_type{});
   if (!PRE && rope) load_rope_cs(p, row0 + lrow, lane, cs0);
   if (p.row_ss) rn.finish(p, rs);
   lds_barrier();

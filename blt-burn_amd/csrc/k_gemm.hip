@@ -64,7 +64,8 @@ int run_gemm_pipe_epi(GemmArgs a, hipStream_t s) {
     case EPI_F32: return run_gemm_pipe<BM, BN, WM, WN, NL, S, EPI_F32>(a, s);
     case EPI_RESID_F32:
       // four waves of 32 x 32 pieces instead of two of 32 x 64: half the MFMA
-      // chain per K tile (M = 48, K = 2048: 9.9 -> 8.6 us; K = 768: 6.2 -> 5.5)
+      // chain per K tile (M = 48, K = 2048: 9.9 -> 8.6 us; K = 768: 6.2 -> 5.5;
+      // 8.2 and 5.3 with the fragment reads across K tiles)
       if constexpr (BM == 64 && BN == 64)
         return run_gemm_pipe<64, 64, 2, 2, 4, S, EPI_RESID_F32>(a, s);
       else
@@ -81,12 +82,12 @@ int run_gemm_pipe_epi(GemmArgs a, hipStream_t s) {
 //   fix + c (k KT + e) + (n / CUs) (kf KT + r)
 // e per tile for the epilogue of its class (residual, other), the last term the
 // memory traffic that grows with the whole launch (r: the residual's).  The
-// constants are least-squares fits to the measured times of the four projection
-// shapes of the model (N, K = 2304, 768; 768, 768; 4096, 768; 768, 2048) at M = 16
-// .. 40000; over those launches the tile it picks is within 7 % of the best
-// (mean 0.4 %).  Measured us (256 x 256 | picked), N = 768, K = 2048: M = 48: 46.7 |
-// 8.6 (64 x 64); 2048: 52.5 | 14.7 (64 x 128); 4096: 50.1 | 20.1 (128 x 128); 8192:
-// 52.4 | 32.4 (128 x 256); 40000: 143 | 143 (128 x 256: 154).  All tiles give
+// constants are fits to the measured times of the four projection shapes of the
+// model (N, K = 2304, 768; 768, 768; 4096, 768; 768, 2048) at M = 16 .. 40000; over
+// those launches the tile it picks is within 6 % of the best (mean 0.2 %).
+// Measured us (256 x 256 | picked), N = 768, K = 2048: M = 48: 47.1 | 8.2 (64 x
+// 64); 2048: 52.4 | 15.4 (64 x 128); 4096: 53.0 | 20.5 (128 x 128); 8192: 55.1 |
+// 31.2 (128 x 256); 40000: 157 | 157 (128 x 256: 156).  All tiles give
 // bit-identical results, so the choice is free of M.
 enum Tile { T64x64, T64x128, T128x128, T128x256, T256x256 };
 struct TileCost {
@@ -94,11 +95,11 @@ struct TileCost {
   double fix, k, e_resid, e_other, kf, r;
 };
 constexpr TileCost kTileCost[] = {
-    {64, 64, 3.263, 0.151, 0.358, 0.716, 0.008, 0.837},
-    {64, 128, 3.124, 0.264, 0.642, 0.425, 0.024, 1.067},
-    {128, 128, 1.030, 0.341, 3.705, 3.510, 0.071, 3.861},
-    {128, 256, 0.182, 0.558, 6.278, 6.044, 0.120, 6.608},
-    {256, 256, 2.072, 1.178, 8.411, 6.376, 0.304, 7.037},
+    {64, 64, 3.288, 0.153, 0.184, 0.561, 0.027, 1.501},
+    {64, 128, 3.824, 0.261, 0.000, 0.001, 0.033, 2.355},
+    {128, 128, 0.434, 0.305, 4.394, 3.868, 0.168, 3.480},
+    {128, 256, 0.000, 0.463, 7.835, 6.446, 0.186, 3.150},
+    {256, 256, 2.954, 1.303, 5.631, 5.373, 0.169, 21.205},
 };
 // a consumer of norm partials on 256 x 256 tiles needs the row_rstd launch
 constexpr double kRowFactorLaunch = 4.5;
@@ -106,7 +107,7 @@ Tile pick_tile(int64_t M, int64_t N, int64_t K, bool resid, bool norm) {
   const int cus = device_cus() > 0 ? device_cus() : 256;
   const double KT = (double)(K / 64);
   const int64_t nb256 = ((M + 255) / 256) * (N / 256);
-  if (nb256 >= 8 * (int64_t)cus) return T256x256;  // its rounds fill the chip
+  if (nb256 >= 4 * (int64_t)cus) return T256x256;  // its rounds fill the chip
   double best = 0;
   Tile t = T256x256;
   for (int i = 0; i < 5; ++i) {
