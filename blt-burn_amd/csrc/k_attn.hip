@@ -459,12 +459,12 @@ int run_attention(const AttnArgs& a, hipStream_t s) {
 // tile's K under its PV MFMAs); the waves of a block read neighbouring tiles, and
 // the blocks of one head share an XCD's L2.
 // Measured us, before (32-query blocks whose threads formed dot products from
-// LDS on the VALU) and now: B = 2, H = 12, T = 1000, d = 64, causal 994 -> 53;
+// LDS on the VALU) and now: B = 2, H = 12, T = 1000, d = 64, causal 998 -> 48;
 // B = 4, H = 12, T = 2048, d = 64, full 6720 -> 590 (87 TFLOP/s); B = 1, H = 4, T
 // = 2048, d = 128, causal 2310 -> 78.  Without its K and V loads the full case
 // takes 390 us: what is left is the loads, K's 32 rows x 32 bytes per
 // instruction above all.  The largest error against 64 bits is no larger than
-// the VALU kernel's (2.6e-7 against 3.3e-7 rel on the first case).
+// the VALU kernel's (2.0e-7 against 3.2e-7 rel on the first case).
 constexpr int F_MAXD = 256;
 
 // ROW: how rows are read: 2 = d is 32 ND, 16-byte rows; 1 = d % 4 == 0, 16-byte
@@ -483,7 +483,7 @@ __global__ __launch_bounds__(256) void attn_f32_kernel(const float* __restrict__
   // a whole V tile in registers beside K's, where that leaves two waves per SIMD
   constexpr bool VPRE = ROW == 2 ? ND <= 4 : ND <= 2;
   __shared__ __attribute__((aligned(16))) float so[NW * 32 * OP];
-  __shared__ float sm[NW][32], sl[NW][32];
+  __shared__ float sm[NW][32], sl[NW][32], sn[32];
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l31 = lane & 31, h = lane >> 5;
@@ -583,16 +583,23 @@ __global__ __launch_bounds__(256) void attn_f32_kernel(const float* __restrict__
       for (int n = 0; n < NV; ++n) load_v(n, vf[n]);
     }
     __builtin_amdgcn_sched_barrier(0);
-    f32x16_t s;
+    // two chains of alternate chunks: half the terms, so less rounding, in each, in
+    // the same time (T = 1000, d = 64: 2.6e-7 -> 2.0e-7 rel against 64 bits; T = 39:
+    // 1.48e-7 -> 1.11e-7)
+    f32x16_t s, s1;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) s[r] = 0.f;
+    for (int r = 0; r < 16; ++r) s[r] = s1[r] = 0.f;
 #pragma unroll
     for (int j = 0; j < NC; ++j)
       if (ROW == 2 || j < NC - 7 || j < nc) {  // chunks wholly past d hold zeros
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-          s = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[j][e], qf[j][e], s, 0, 0, 0);
+        for (int e = 0; e < 4; ++e) {
+          f32x16_t& c = j & 1 ? s1 : s;
+          c = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[j][e], qf[j][e], c, 0, 0, 0);
+        }
       }
+#pragma unroll
+    for (int r = 0; r < 16; ++r) s[r] += s1[r];
     __builtin_amdgcn_sched_barrier(0);
     // (unconditional, so the wait for V below leaves these loads in flight; after
     // the wave's last tile they re-read one of its rows)
@@ -675,8 +682,10 @@ __global__ __launch_bounds__(256) void attn_f32_kernel(const float* __restrict__
   float lt = 0.f;
 #pragma unroll
   for (int i = 0; i < NW; ++i) lt += sl[i][l31] * expw(sm[i][l31] - mu);
-  // a query that sees no key gets 0
-  const float f = lt > 0.f ? wt / lt : 0.f;
+  // The sum of the weighted partials is divided once at the end, not each of them
+  // times a rounded factor (T = 3, d = 64: 5.4e-8 -> 5.2e-8 rel against 64 bits).
+  // A query that sees no key gets 0.
+  if (w == 0 && h == 0) sn[l31] = lt > 0.f ? lt : INFINITY;
   float* orow = so + (w * 32 + l31) * OP;
 #pragma unroll
   for (int n = 0; n < NV; ++n)
@@ -684,7 +693,7 @@ __global__ __launch_bounds__(256) void attn_f32_kernel(const float* __restrict__
     for (int r = 0; r < 16; ++r) {
       vf_t x;
 #pragma unroll
-      for (int u = 0; u < VW; ++u) x[u] = oacc[n * VW + u][r] * f;
+      for (int u = 0; u < VW; ++u) x[u] = oacc[n * VW + u][r] * wt;
       *reinterpret_cast<vf_t*>(orow + VW * (8 * (r >> 2) + 4 * h + (r & 3)) + 32 * VW * n) = x;
     }
   __syncthreads();
@@ -694,7 +703,7 @@ __global__ __launch_bounds__(256) void attn_f32_kernel(const float* __restrict__
   for (int i = tid; i < nq * d; i += 256) {
     const int r = i / d, c = i - r * d;
     const float* p = so + r * OP + c;
-    dst[i] = (p[0] + p[32 * OP]) + (p[64 * OP] + p[96 * OP]);
+    dst[i] = ((p[0] + p[32 * OP]) + (p[64 * OP] + p[96 * OP])) / sn[r];
   }
 }
 
