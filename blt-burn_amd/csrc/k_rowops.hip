@@ -715,6 +715,7 @@ __global__ __launch_bounds__(PB_THREADS) void patch_boundary_kernel(
 // element of the longest chain.  [16, 8192], patches of 8 on average: 27 us with
 // one block per row walking its tiles, 8 us now; one row of 8,000 that is a single
 // patch: 70 us with one lane adding both signals in turn, 31 us now.
+// Rows that one block has to walk take patch_means_walk_kernel.
 // ---------------------------------------------------------------------------
 constexpr int PM_THREADS = 256;
 constexpr int PM_TILE = 1024;
@@ -775,8 +776,7 @@ __global__ __launch_bounds__(PM_THREADS) void patch_means_kernel(
   const int64_t roff = row_off ? row_off[b] : b * T_dense;
   const int64_t T = row_len ? (int64_t)row_len[b] : T_dense;
   const int64_t ooff = out_off ? out_off[b] : roff;
-  // without starts every row is one patch [0, T)
-  int64_t n = starts ? (int64_t)count[b] : 1;
+  int64_t n = count[b];
   n = n < 0 ? 0 : (n > T ? T : n);
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
   auto in = [&](int a) { return a == 0 ? H : a == 1 ? N : C; };
@@ -790,7 +790,7 @@ __global__ __launch_bounds__(PM_THREADS) void patch_means_kernel(
   auto span = [&](int64_t p, int64_t& st, int64_t& e) {
     e = p + 1 < n ? (int64_t)starts[roff + p + 1] : T;
     e = e < 0 ? 0 : (e > T ? T : e);
-    st = starts ? (int64_t)starts[roff + p] : 0;
+    st = starts[roff + p];
     st = st < 0 ? 0 : (st > e ? e : st);
   };
   auto put = [&](int a, int64_t p, float sum, int64_t len) {
@@ -808,7 +808,7 @@ __global__ __launch_bounds__(PM_THREADS) void patch_means_kernel(
     while (lo < hi) {
       const int64_t step = (hi - lo + PM_THREADS - 1) / PM_THREADS;
       const int64_t p = lo + tid * step;
-      const bool below = p < hi && (starts ? starts[roff + p] : 0) < t0;
+      const bool below = p < hi && starts[roff + p] < t0;
       const uint64_t bal = __ballot(below);
       if (lane == 0) probes[wid] = __popcll(bal);
       __syncthreads();
@@ -866,6 +866,154 @@ __global__ __launch_bounds__(PM_THREADS) void patch_means_kernel(
       if (wid == 0 && lane < NA) put(lane, p, sum, e - st);
     }
     __syncthreads();  // the buffers and run_* are reused by the block's next tile
+  }
+}
+
+// The same means by one block per row, tile after tile in order: for rows without
+// starts (one chain) and for means that overlap an input, where a tile's means may
+// be written only once every earlier position has been read (patch p starts at p or
+// later, so its mean lands at a position that this block is past).  A lane takes all
+// signals of a short patch (a tile of them is one round of the block, where a lane
+// per signal is three) and one signal of a long one.  The patch that runs past a
+// tile's end hands its sums on.  The next tile's positions are loaded under the
+// current one's chains, and a tile's first patch is known from the tile before.
+// What bounds it is the read of the tile's starts, a barrier and the longest chain.
+// Measured us in place, coherence included, with a kernel that searched each
+// tile's first start and staged what ran past its end twice, and now: [16, 8192] in
+// patches of 8: 45 -> 19; [1, 131072]: 718 -> 244; as one patch: 638 -> 473.
+constexpr int PW_TILE = 2048;
+constexpr int PW_LONG = 96;  // at most 21 patches of a tile are longer: a wave holds their signals
+template <int NA>
+__global__ __launch_bounds__(PM_THREADS) void patch_means_walk_kernel(
+    const float* H, const float* N, const float* C, const int32_t* __restrict__ starts,
+    const int32_t* __restrict__ count, int64_t T_dense, const int64_t* __restrict__ row_off,
+    const int32_t* __restrict__ row_len, float* mH, float* mN, float* mC,
+    const int64_t* __restrict__ out_off) {
+  constexpr int PER = PW_TILE / 4 / PM_THREADS;  // 4-position pieces per thread and signal
+  typedef float piece_t __attribute__((ext_vector_type(4), aligned(4)));  // (rows start anywhere)
+  // what one tile hands to the next alternates between two copies, so one barrier
+  // per tile is enough
+  __shared__ __attribute__((aligned(16))) float sx[2][NA][PW_TILE + 4];
+  __shared__ float run_s[2][NA];  // sums of the patch that runs on
+  __shared__ int long_of[PM_THREADS / 64][64];  // lanes of a wave that hold a long patch
+  // the tile's last patch, with its span and the tile it was written for
+  __shared__ int64_t end_p[2], end_st[2], end_e[2], end_t0[2];
+  const int64_t b = blockIdx.x;
+  const int64_t roff = row_off ? row_off[b] : b * T_dense;
+  const int64_t T = row_len ? (int64_t)row_len[b] : T_dense;
+  const int64_t ooff = out_off ? out_off[b] : roff;
+  // without starts the row is one patch [0, T)
+  int64_t n = starts ? (int64_t)count[b] : 1;
+  n = n < 0 ? 0 : (n > T ? T : n);
+  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  f32x4_t pre[NA][PER];
+  auto load = [&](int64_t t0) {
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int64_t t = t0 + 4 * (tid + i * PM_THREADS);
+#pragma unroll
+      for (int a = 0; a < NA; ++a) {
+        const float* x = (a == 0 ? H : a == 1 ? N : C) + roff;
+        if (t + 4 <= T) {
+          pre[a][i] = *reinterpret_cast<const piece_t*>(x + t);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) pre[a][i][e] = t + e < T ? x[t + e] : 0.f;
+        }
+      }
+    }
+  };
+  // patch p's span, clamped to 0 <= st <= e <= T
+  auto span = [&](int64_t p, int64_t& st, int64_t& e) {
+    e = p + 1 < n ? (int64_t)starts[roff + p + 1] : T;
+    e = e < 0 ? 0 : (e > T ? T : e);
+    st = starts ? (int64_t)starts[roff + p] : 0;
+    st = st < 0 ? 0 : (st > e ? e : st);
+  };
+  if (tid < 2) end_t0[tid] = -1;
+  load(0);
+  int64_t lo = 0;  // first patch that has not started in an earlier tile
+  int k = 0;
+  for (int64_t t0 = 0; t0 < T; t0 += PW_TILE, k ^= 1) {
+    const int64_t t1 = t0 + PW_TILE < T ? t0 + PW_TILE : T;
+    const bool last_tile = t1 == T;
+#pragma unroll
+    for (int a = 0; a < NA; ++a)
+#pragma unroll
+      for (int i = 0; i < PER; ++i)
+        *reinterpret_cast<f32x4_t*>(&sx[k][a][4 * (tid + i * PM_THREADS)]) = pre[a][i];
+    __syncthreads();
+    int64_t rst = 0, re = 0;  // the span of the patch that goes on into this tile
+    if (t0 > 0 && end_t0[k ^ 1] == t0 - PW_TILE) {
+      lo = end_p[k ^ 1] + 1;
+      rst = end_st[k ^ 1];
+      re = end_e[k ^ 1];
+    }
+    if (lo >= n && re <= t0) break;
+    // patch p's sums end at e: written, or handed on
+    auto finish = [&](int a, int64_t p, int64_t st, int64_t e, float sum) {
+      float* m = a == 0 ? mH : a == 1 ? mN : mC;
+      if (e > t1) run_s[k][a] = sum;
+      else if (m) m[ooff + p] = e > st ? sum / (float)(e - st) : 0.f;
+      if (a == 0 && e >= t1) {  // the tile's last patch
+        end_p[k] = p;
+        end_st[k] = st;
+        end_e[k] = e;
+        end_t0[k] = t0;
+      }
+    };
+    int64_t p = lo + tid, st = T, e = T;
+    if (p < n) span(p, st, e);  // (ahead of the next tile's loads)
+    if (!last_tile) load(t1);
+    if (re > t0 && tid < NA)
+      finish(tid, lo - 1, rst, re,
+             pm_chain(sx[k][tid], 0, (int)((re < t1 ? re : t1) - t0), run_s[k ^ 1][tid]));
+    for (int64_t p0 = lo;; p0 += PM_THREADS) {
+      // starts ascend: past one that lies further on, so do all
+      bool mine = p < n && (last_tile || st < t1);
+      if (!__any(mine)) break;
+      // (st < t0 only for starts that do not ascend)
+      int t = (int)((st < t0 ? t0 : st > t1 ? t1 : st) - t0);
+      const int z = (int)((e < t1 ? (e < t0 ? t0 : e) : t1) - t0);
+      // the wave's long patches, a lane per signal
+      const uint64_t lm = __ballot(mine && z - t >= PW_LONG);
+      if (lm) {
+        const int rank = __popcll(lm & ((1ull << lane) - 1));
+        const bool is_long = (lm >> lane) & 1 && rank < 64 / NA;
+        if (is_long) long_of[wid][rank] = lane;
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // (the wave's own writes)
+        const int m = __popcll(lm) < 64 / NA ? __popcll(lm) : 64 / NA;
+        const int a = lane % NA, from = lane / NA < m ? long_of[wid][lane / NA] : 0;
+        const int lt = __shfl(t, from), lz = __shfl(z, from);
+        const int64_t lst = __shfl(st, from), le = __shfl(e, from);
+        if (lane / NA < m)
+          finish(a, p0 + wid * 64 + from, lst, le, pm_chain(sx[k][a], lt, lz, 0.f));
+        mine = mine && !is_long;
+      }
+      if (mine) {
+        float sum[NA];
+#pragma unroll
+        for (int a = 0; a < NA; ++a) sum[a] = 0.f;
+        auto one = [&] {
+#pragma unroll
+          for (int a = 0; a < NA; ++a) sum[a] += sx[k][a][t];
+          ++t;
+        };
+        while (t < z && (t & 3)) one();
+#pragma unroll 4
+        for (; t + 4 <= z; t += 4)
+#pragma unroll
+          for (int a = 0; a < NA; ++a) {
+            const f32x4_t x = *reinterpret_cast<const f32x4_t*>(&sx[k][a][t]);
+            sum[a] += x.x; sum[a] += x.y; sum[a] += x.z; sum[a] += x.w;
+          }
+        while (t < z) one();
+#pragma unroll
+        for (int a = 0; a < NA; ++a) finish(a, p, st, e, sum[a]);
+      }
+      p += PM_THREADS;
+      if (p < n) span(p, st, e);
+    }
   }
 }
 
@@ -1244,26 +1392,22 @@ int launch_patch_means(const float* H, const float* N, const float* C, const int
                        const int32_t* row_len, int64_t max_len, float* mH, float* mN, float* mC,
                        hipStream_t s, const int64_t* out_off) {
   if (B == 0) return 0;
-  // one block per tile; a row without starts is one chain, so one block.  A
-  // caller's mean that overlaps an input keeps one block per row: it has read a
-  // position before it writes a mean there (patch p starts at p or later).
-  int64_t tiles = starts ? ((row_len ? max_len : T) + PM_TILE - 1) / PM_TILE : 1;
-  if (!row_len) {
+  // One block per tile.  A row without starts is one chain, and a caller's mean
+  // that overlaps an input has to keep the order of one walk: one block per row.
+  bool walk = !starts;
+  if (!row_len && T > PM_TILE) {
     auto overlap = [&](const float* m, const float* x) {
       return m && x && m < x + B * T && x < m + B * T;
     };
     for (const float* m : {mH, mN, mC})
-      for (const float* x : {H, N, C})
-        if (overlap(m, x)) tiles = 1;
+      for (const float* x : {H, N, C}) walk = walk || overlap(m, x);
   }
-  tiles = tiles < 1 ? 1 : tiles > 65535 ? 65535 : tiles;
-  const dim3 grid((unsigned)B, (unsigned)tiles);
-  if (C)
-    hipLaunchKernelGGL(patch_means_kernel<3>, grid, dim3(PM_THREADS), 0, s, H, N, C, starts, count,
-                       T, row_off, row_len, mH, mN, mC, out_off);
-  else
-    hipLaunchKernelGGL(patch_means_kernel<2>, grid, dim3(PM_THREADS), 0, s, H, N, C, starts, count,
-                       T, row_off, row_len, mH, mN, mC, out_off);
+  const int64_t tiles = ((row_len ? max_len : T) + PM_TILE - 1) / PM_TILE;
+  const dim3 grid((unsigned)B, walk || tiles < 1 ? 1 : tiles > 65535 ? 65535 : (unsigned)tiles);
+  auto kern = walk ? (C ? patch_means_walk_kernel<3> : patch_means_walk_kernel<2>)
+                   : (C ? patch_means_kernel<3> : patch_means_kernel<2>);
+  hipLaunchKernelGGL(kern, grid, dim3(PM_THREADS), 0, s, H, N, C, starts, count, T, row_off,
+                     row_len, mH, mN, mC, out_off);
   BLT_LAUNCH_CHECK("patch_means_kernel");
   return 0;
 }

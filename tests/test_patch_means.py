@@ -109,8 +109,8 @@ def test_device_bit_exact_vs_oracle():
 @pytest.mark.gpu
 @pytest.mark.parametrize("T", [5000, 8192, 20000])
 def test_device_long_patches_bit_exact(T):
-    """Patches longer than the kernel's 2048-position LDS tiles (their sums
-    carried from tile to tile), patches ending or starting exactly on tile
+    """Patches longer than the kernel's 1024-position LDS tiles (their sums
+    carried on past the tile), patches ending or starting exactly on tile
     edges, and one patch over the whole row, bit-exact against the oracle."""
     import torch
     from blt_burn_amd import patcher
@@ -166,6 +166,64 @@ def test_device_means_at_tile_edges_bit_exact(T):
             assert np.array_equal(mN.cpu().numpy()[b, :k], rN[b, :k]), (T, b)
             if C is not None:
                 assert np.array_equal(mC.cpu().numpy()[b, :k], rC[b, :k]), (T, b)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T", [1024, 1025, 2048, 5000, 9216])
+def test_device_means_in_place_bit_exact(T):
+    """Means written over all three inputs: one block walks the row's tiles, a
+    patch's sums go from tile to tile.  Patches over whole tiles without a start,
+    ends and starts on and beside tile edges, tiles of one-position patches (more
+    of them than threads), a first start inside a later tile, a start past the row
+    end, and no patch at all."""
+    import torch
+    from blt_burn_amd import patcher
+    rng = np.random.default_rng(T)
+    edges = [t for e in range(1024, T, 1024) for t in (e - 1, e, e + 1) if t < T]
+    rows = [[0], [], list(range(T)), [0] + edges, [0] + list(range(1024, T, 1024)),
+            [0] + [t for t in (7, 1023, 4096) if t < T], [t for t in (1024, 3500) if t < T],
+            [0] + list(range(max(1, T - 1500), T)), [0, T - 1, T + 5],
+            [0] + sorted(rng.choice(np.arange(1, T), T // 9, replace=False).tolist())]
+    B = len(rows)
+    H = rng.normal(3.0, 1.0, (B, T)).astype(np.float32)
+    N = (rng.random((B, T)) * 30).astype(np.float32)
+    C = (N * N / (H + 1e-6)).astype(np.float32)
+    st, ct = _starts(rows, T)
+    ref = oracle.patch_means(H, N, st, ct, C)
+    sd, cd = torch.from_numpy(st).cuda(), torch.from_numpy(ct).cuda()
+    for perm in ((0, 1, 2), (1, 2, 0)):  # each mean over its own input, over another
+        x = [torch.from_numpy(a).cuda() for a in (H, N, C)]
+        out = patcher.patch_means(x[0], x[1], sd, cd, x[2], out=[x[i] for i in perm])
+        for got, want in zip(out, ref):
+            got = got.cpu().numpy()
+            for b in range(B):
+                assert np.array_equal(got[b, :ct[b]], want[b, :ct[b]]), (T, b, perm)
+
+
+@pytest.mark.gpu
+def test_device_means_in_place_walk_time():
+    """A walk visits each tile once: [1, 131072] in patches of 8 on average, means
+    over their inputs, in less than 3 us per 1024 positions (a tile needs one
+    barrier, one dependent read of its starts and a short chain; searching for its
+    first start and staging what lies past its end again took 5.6 us)."""
+    import torch
+    from blt_burn_amd import patcher
+    T = 131072
+    rng = np.random.default_rng(8)
+    rows = [[0] + sorted(rng.choice(np.arange(1, T), T // 8, replace=False).tolist())]
+    sd, cd = (torch.from_numpy(a).cuda() for a in _starts(rows, T))
+    x = [torch.rand(1, T, device="cuda") for _ in range(3)]
+    ev = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+    us = []
+    for _ in range(6):
+        ev[0].record()
+        for _ in range(5):
+            patcher.patch_means(x[0], x[1], sd, cd, x[2], out=x)
+        ev[1].record()
+        torch.cuda.synchronize()
+        us.append(ev[0].elapsed_time(ev[1]) * 200)
+    print("patch_means in place [1, %d]: %.0f us" % (T, min(us)))
+    assert min(us) < 3.0 * T / 1024, us
 
 
 @pytest.mark.gpu
