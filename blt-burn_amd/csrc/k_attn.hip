@@ -467,8 +467,18 @@ int run_attention(const AttnArgs& a, hipStream_t s) {
 // the VALU kernel's (2.0e-7 against 3.2e-7 rel on the first case).
 constexpr int F_MAXD = 256;
 
-// ROW: how rows are read: 2 = d is 32 ND, 16-byte rows; 1 = d % 4 == 0, 16-byte
-// rows; 0 = element by element.
+// ROW: how rows are read: 2 = d is 32 ND and every tensor 16-byte aligned; 1 = d % 4
+// == 0, in 16-byte pieces too, which global loads take at any 4-byte address; 0 = any
+// other d: pieces past the row's end are cut out of its last 16 bytes (d < 32, which
+// need not have them: element by element), V is read a column at a time.
+template <int W, bool ALIGNED>
+struct FVec {
+  typedef float type __attribute__((ext_vector_type(W)));
+};
+template <int W>
+struct FVec<W, false> {
+  typedef float type __attribute__((ext_vector_type(W), aligned(4)));
+};
 template <int ND, int ROW>
 __global__ __launch_bounds__(256) void attn_f32_kernel(const float* __restrict__ q,
                                                        const float* __restrict__ k,
@@ -480,8 +490,16 @@ __global__ __launch_bounds__(256) void attn_f32_kernel(const float* __restrict__
   auto expw = [&](float x) { return __builtin_amdgcn_exp2f(x * cs); };
   constexpr int NW = 4, NC = 4 * ND;     // waves; 8-wide chunks of the head dim
   constexpr int OP = 32 * ND + 4;        // output row pitch in LDS (floats)
-  // a whole V tile in registers beside K's, where that leaves two waves per SIMD
+  // A whole V tile in registers beside K's, where they fit: two waves per SIMD up to
+  // d = 64, one above (a second one, of 248 registers at d = 96, was no gain: [1, 12,
+  // 1024, 96] causal 42 us with one wave, 70 with two, whose blocks share a CU while
+  // others idle).
   constexpr bool VPRE = ROW == 2 ? ND <= 4 : ND <= 2;
+  // Where the row pitch is no constant, V's addresses are a uniform row base and a lane
+  // offset that the compiler may not take for a constant of the key loop: it would
+  // keep the sums of all rows and column blocks in registers, and spill from d = 129
+  // on.  With few of them (ND = 1, or 2 in 16-byte rows) that is the faster form.
+  constexpr bool OPAQUE = ROW == 0 ? ND > 1 : ROW == 1 && ND > 2;
   __shared__ __attribute__((aligned(16))) float so[NW * 32 * OP];
   __shared__ float sm[NW][32], sl[NW][32], sn[32];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -503,17 +521,28 @@ __global__ __launch_bounds__(256) void attn_f32_kernel(const float* __restrict__
   const float* kb = k + bh * Tkv * d;
   const float* vb = v + bh * Tkv * d;
   const int nc = (d + 7) / 8;
+  // chunks that lie wholly in a row of the instantiation's smallest d (ND = 6 and 8
+  // serve 64 of them)
+  constexpr int WHOLE = ND > 4 ? NC - 8 : NC - 4;
+  using piece_t = typename FVec<4, ROW == 2>::type;
 
   // the lane's pieces of one row: elements 8 j + 4 h .. + 3, zero past d
   auto load_row = [&](const float* row, f32x4_t (&f)[NC]) {
 #pragma unroll
     for (int j = 0; j < NC; ++j) {
       const int c = 8 * j + 4 * h;
-      if constexpr (ROW == 2) {
-        f[j] = *reinterpret_cast<const f32x4_t*>(row + c);
-      } else if constexpr (ROW == 1) {
-        const f32x4_t x = *reinterpret_cast<const f32x4_t*>(row + (c < d ? c : 0));
+      if (ROW == 2 || j < WHOLE) {
+        f[j] = *reinterpret_cast<const piece_t*>(row + c);
+      } else if (ROW == 1) {
+        const f32x4_t x = *reinterpret_cast<const piece_t*>(row + (c < d ? c : 0));
         f[j] = c < d ? x : f32x4_t{0.f, 0.f, 0.f, 0.f};
+      } else if (ND > 1) {
+        // the row's last four elements, moved down by how far they lie before c
+        const int at = c < d - 4 ? c : d - 4, sh = c - at;
+        f32x4_t x = *reinterpret_cast<const piece_t*>(row + at);
+        x = sh & 1 ? f32x4_t{x.y, x.z, x.w, 0.f} : x;
+        x = sh & 2 ? f32x4_t{x.z, x.w, 0.f, 0.f} : x;
+        f[j] = sh < 4 ? x : f32x4_t{0.f, 0.f, 0.f, 0.f};
       } else {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -539,7 +568,8 @@ __global__ __launch_bounds__(256) void attn_f32_kernel(const float* __restrict__
   // % VW + 32 VW (n / VW).  Columns past d: rows of O^T that are never stored.
   constexpr int VW = ROW == 0 ? 1 : ND % 4 == 0 ? 4 : ND % 2 == 0 ? 2 : 1;
   constexpr int NV = ND / VW;
-  typedef float vf_t __attribute__((ext_vector_type(VW)));
+  using vf_t = typename FVec<VW, true>::type;
+  using vp_t = typename FVec<VW, ROW == 2>::type;
   int dcol[NV];
 #pragma unroll
   for (int n = 0; n < NV; ++n) {
@@ -562,17 +592,24 @@ __global__ __launch_bounds__(256) void attn_f32_kernel(const float* __restrict__
     const int last = PART ? (int)(Tkv - 1 - k0) : 31;  // the tile's last valid key
     // V of key k0 + 8 (r / 4) + 4 h + r % 4; zero past Tkv
     auto load_v = [&](int n, vf_t (&f)[16]) {
+      unsigned off = 0;
+      if constexpr (OPAQUE && !PART) {
+        off = (unsigned)(4 * h * dd + dcol[n]);
+        asm volatile("" : "+v"(off));
+      }
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int kr = 8 * (r >> 2) + (r & 3);
         if constexpr (PART) {
           const int key = kr + 4 * h;
-          const vf_t x = *reinterpret_cast<const vf_t*>(
+          const vf_t x = *reinterpret_cast<const vp_t*>(
               vt + (unsigned)((key < last ? key : last) * dd + dcol[n]));
 #pragma unroll
           for (int u = 0; u < VW; ++u) f[r][u] = key <= last ? x[u] : 0.f;
+        } else if constexpr (OPAQUE) {
+          f[r] = *reinterpret_cast<const vp_t*>(vt + (int64_t)kr * dd + off);
         } else {
-          f[r] = *reinterpret_cast<const vf_t*>(
+          f[r] = *reinterpret_cast<const vp_t*>(
               vt + ((unsigned)(4 * h * dd + dcol[n]) + (unsigned)(kr * dd)));
         }
       }
@@ -712,12 +749,12 @@ int run_attention_f32(const float* q, const float* k, const float* v, float* o, 
                       int64_t H, int64_t Tq, int64_t Tkv, int d, int causal, hipStream_t s) {
   const dim3 grid((unsigned)((Tq + 31) / 32), (unsigned)H, (unsigned)B);
   const float cs = (float)(1.44269504088896340736 / sqrt((double)d));
-  const bool vec = d % 4 == 0 && (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v) & 15) == 0;
   // heads whose K and V share half an XCD's 4 MB L2, at most an eighth of them
   const int64_t fit = (int64_t)(2 << 20) / (Tkv * d * 8 + 1), share = (B * H + 7) / 8;
   const int hgroup = (int)(fit < 1 ? 1 : fit < share ? fit : share);
-  auto kern = !vec ? attn_f32_kernel<ND, 0>
-                   : d == 32 * ND ? attn_f32_kernel<ND, 2> : attn_f32_kernel<ND, 1>;
+  const bool al16 = (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v) & 15) == 0;
+  auto kern = d % 4 ? attn_f32_kernel<ND, 0>
+                   : d == 32 * ND && al16 ? attn_f32_kernel<ND, 2> : attn_f32_kernel<ND, 1>;
   hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, q, k, v, o, Tq, Tkv, d, causal ? 1 : 0, hgroup,
                      cs);
   BLT_LAUNCH_CHECK("attn_f32_kernel");

@@ -124,7 +124,7 @@ int blt_fused_attention_bf16(const uint16_t* q, const uint16_t* k, const uint16_
  * (attention_kernel.rs:20-125, launched by backend.rs:334-383): q [B, H, Tq, d],
  * k and v [B, H, Tkv, d], o [B, H, Tq, d], all f32, dense head-major; any
  * head_dim d <= 256; causal: key j visible to query i iff j <= i.  Scores
- * (q . k) / sqrt(d) and the softmax in f32 on the VALU (no bf16 rounding); a
+ * (q . k) / sqrt(d) and the softmax in f32 throughout (no bf16 rounding); a
  * query that sees no key gets 0.  blt_fused_attention_bf16 is the MFMA path
  * (d = 64, RoPE and windows) the model uses. */
 int blt_fused_attention_f32(const float* q, const float* k, const float* v, float* o, int64_t B,

@@ -536,6 +536,63 @@ def test_attention_f32_tile_edges(d):
     assert torch.all(o == 0.0)
 
 
+@pytest.mark.parametrize("d", [33, 34, 35, 66, 97, 127, 130, 131, 161, 191, 193, 226, 255])
+def test_attention_f32_row_tails(d):
+    # d % 4 != 0 above 32: the last piece of a row is cut out of its last 16
+    # bytes, at every remainder and every instantiation's smallest and largest
+    # d; the bound is the test's above.  Tensors that start 4, 8 or 12 bytes
+    # past a 16-byte address give the same bits.
+    L = _lib.lib()
+    stream = torch.cuda.current_stream().cuda_stream
+    Tq, Tkv = 40, 70
+    q, k, v = (synth.normal_f32(i + d, (1, 2, n, d))
+               for i, n in ((311, Tq), (312, Tkv), (313, Tkv)))
+    ref = oracle.attention_kernel(q, k, v, True)
+    first = None
+    for shift in (0, 1, 2, 3):
+        dev = []
+        for x in (q, k, v):
+            buf = torch.full((x.size + shift + 4,), float("nan"), device=DEV)  # (no stray reads)
+            buf[shift:shift + x.size] = torch.from_numpy(x.reshape(-1))
+            dev.append(buf[shift:])
+        o = torch.empty(q.size, device=DEV)
+        _lib.check(L.blt_fused_attention_f32(*[t.data_ptr() for t in dev], o.data_ptr(), 1, 2, Tq,
+                                             Tkv, d, 1, stream), "attention_f32")
+        torch.cuda.synchronize()
+        np.testing.assert_allclose(o.cpu().numpy().reshape(ref.shape), ref, atol=5e-5, rtol=0,
+                                   err_msg=str(shift))
+        first = o if first is None else first
+        assert torch.equal(o, first), shift
+
+
+def test_attention_f32_every_row_form_time():
+    # rows of any length and alignment are read in 16-byte pieces and none of
+    # the forms spills: [1, 4, 33, 33] at d = 225, and at d = 256 from a 4-byte
+    # address, within twice the aligned d = 256 call (element by element, and
+    # with spilled addresses, they took 4.6 times it)
+    L = _lib.lib()
+    stream = torch.cuda.current_stream().cuda_stream
+    x = [torch.randn(4 * 33 * 256 + 4, device=DEV) for _ in range(4)]
+    ev = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+
+    def us(d, shift):
+        best = 1e9
+        for _ in range(6):
+            ev[0].record()
+            for _ in range(20):
+                _lib.check(L.blt_fused_attention_f32(*[t[shift:].data_ptr() for t in x], 1, 4, 33,
+                                                     33, d, 0, stream), "attention_f32")
+            ev[1].record()
+            torch.cuda.synchronize()
+            best = min(best, ev[0].elapsed_time(ev[1]) * 50)
+        return best
+
+    base, tail, off = us(256, 0), us(225, 0), us(256, 1)
+    print("f32 attention: d = 256 %.1f us, d = 225 %.1f, d = 256 misaligned %.1f"
+          % (base, tail, off))
+    assert max(tail, off) < 2 * base, (base, tail, off)
+
+
 def test_attention_f32_rejects_wide_heads():
     q = cuda(synth.normal_f32(90, (1, 1, 8, 264)))
     with pytest.raises(_lib.BltError):
