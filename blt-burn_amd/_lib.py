@@ -85,6 +85,7 @@ EXPORTS = {
                                        c_i32, c_i32, c_i32, c_i64, c_vp, c_vp]),
     "blt_probe_mfma_flops": (c_i64, [c_i32, c_i32]),
     "blt_probe_mfma_bf16": (c_i32, [c_i32, c_i32, c_vp, c_vp]),
+    "blt_gemm_tile": (c_i32, [c_i64, c_i64, c_i64, c_i32]),
     "blt_probe_copy": (c_i32, [c_vp, c_vp, c_i64, c_vp]),
 }
 

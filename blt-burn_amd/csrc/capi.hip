@@ -523,4 +523,11 @@ int blt_gemm_bf16_epilogue(const uint16_t* A, const uint16_t* Bt, void* C, int64
   return launch_gemm(g, STREAM(stream));
 }
 
+int32_t blt_gemm_tile(int64_t M, int64_t N, int64_t K, int32_t epilogue) {
+  if (M <= 0 || N <= 0 || K <= 0 || K % 64 != 0 || epilogue < BLT_EPI_BF16 ||
+      epilogue > BLT_EPI_SILU_GATE)
+    return fail(-2, "gemm_tile: need M, N > 0, K % 64 == 0, an epilogue");
+  return gemm_tile(M, N, K, epilogue);
+}
+
 }  // extern "C"

@@ -20,9 +20,10 @@ int device_cus() {
 template <int BM, int BN, int BK, int WM, int WN, int EPI>
 int run_gemm_persistent(const GemmArgs& a, hipStream_t s) {
   const int64_t nb = ((a.M + BM - 1) / BM) * ((a.N + BN - 1) / BN);
-  // one block per CU (its LDS holds 160 KB), a multiple of 8 blocks so each
+  // as many blocks as fit on the CUs at once (256 x 256: one per CU, its LDS
+  // holds 160 KB; 128 x 128: two, 80 KB each), a multiple of 8 blocks so each
   // keeps its XCD residue
-  int64_t grid = device_cus();
+  int64_t grid = (int64_t)device_cus() * (BM * BN <= 128 * 128 ? 2 : 1);
   grid = grid >= 8 ? grid & ~7 : grid;
   if (grid <= 0 || grid > nb) grid = nb;
   hipLaunchKernelGGL((gemm::gemm_bf16_dma_persistent_kernel<BM, BN, BK, WM, WN, EPI>),
@@ -38,7 +39,11 @@ int run_gemm_dma_epi(const GemmArgs& a, hipStream_t s) {
     case EPI_BF16: return run_gemm_persistent<BM, BN, BK, WM, WN, EPI_BF16>(a, s);
     case EPI_F32: return run_gemm_persistent<BM, BN, BK, WM, WN, EPI_F32>(a, s);
     case EPI_RESID_F32: return run_gemm_persistent<BM, BN, BK, WM, WN, EPI_RESID_F32>(a, s);
-    case EPI_QKV_ROPE: return run_gemm_persistent<BM, BN, BK, WM, WN, EPI_QKV_ROPE>(a, s);
+    case EPI_QKV_ROPE:
+      // (pick_tile gives QKV no persistent 128 x 128 tiles)
+      if constexpr (BM == 256)
+        return run_gemm_persistent<BM, BN, BK, WM, WN, EPI_QKV_ROPE>(a, s);
+      break;
     case EPI_SILU_GATE: return run_gemm_persistent<BM, BN, BK, WM, WN, EPI_SILU_GATE>(a, s);
   }
   return fail(-2, "gemm: unknown epilogue");
@@ -77,49 +82,69 @@ int run_gemm_pipe_epi(GemmArgs a, hipStream_t s) {
 }
 
 // ---- choice of the tile (N % 256 == 0) ---------------------------------------
-// The predicted time of a launch on each tile, in us, with n tiles, c = ceil(n /
-// CUs) of them on the fullest CU and KT K tiles:
-//   fix + c (k KT + e) + (n / CUs) (kf KT + r)
-// e per tile for the epilogue of its class (residual, other), the last term the
-// memory traffic that grows with the whole launch (r: the residual's).  The
-// constants are fits to the measured times of the four projection shapes of the
-// model (N, K = 2304, 768; 768, 768; 4096, 768; 768, 2048) at M = 16 .. 40000; over
-// those launches the tile it picks is within 6 % of the best (mean 0.2 %).
-// Measured us (256 x 256 | picked), N = 768, K = 2048: M = 48: 47.1 | 8.2 (64 x
-// 64); 2048: 52.4 | 15.4 (64 x 128); 4096: 53.0 | 20.5 (128 x 128); 8192: 55.1 |
-// 31.2 (128 x 256); 40000: 157 | 157 (128 x 256: 156).  All tiles give
-// bit-identical results, so the choice is free of M.
-enum Tile { T64x64, T64x128, T128x128, T128x256, T256x256 };
+// The predicted time of a launch on each tile, in us, with n tiles, KT K tiles, f = n
+// / CUs, c1 = ceil(f) and c2 = ceil(f / 2), the rounds of one and of two blocks per CU:
+//   fix + (k1 c1 + k2 c2 + kf f) KT + e c1 + o c2 + r f
+// (k2 and o for the tiles that two blocks of a CU share; e and r by epilogue: the
+// tile's own latency and the part that grows with the whole launch's traffic), and for
+// a launch with row norms norm f where the tile forms the factors itself, else the
+// row_rstd launch.  The constants are fits to 4150 launches on every tile in four
+// runs: M = 1 .. 65536, N = 256 .. 12288, K = 64 .. 4096, every epilogue.  Over the
+// projections of models (residual, and QKV and SiLU with row norms) the tile it picks
+// takes 0.7 % longer than the best of the six on average, 10 % at the 99th percentile;
+// a K or N left out of the fit: 0.2 to 1.3 % on average.  25 of those 1744 launches are
+// over 3 % slower than on the two persistent tiles alone.  (A fit to K = 768 and 2048
+// with one epilogue column for QKV, SiLU and bf16, and without T128x128x2: 1.8 %, 23 %,
+// and 114 of them; a model of dim 256 at [4, 8192] took 366 us against 338.)
+// Measured us (256 x 256 | picked), N = 768, K = 2048: M = 48: 45.5 | 7.7 (64 x 64);
+// 2048: 49.6 | 14.2 (64 x 128); 4096: 51.0 | 20.8 (128 x 128); 8192: 54.7 | 31.5 (128 x
+// 256).  All tiles give bit-identical results, so the choice is free of M.
+enum Tile { T64x64, T64x128, T128x128, T128x256, T256x256, T128x128x2 };
 struct TileCost {
   int bm, bn;
-  double fix, k, e_resid, e_other, kf, r;
+  double fix, k1, k2, kf, o, norm;
+  double e[5], r[5];  // by Epilogue
 };
+// T256x256 and T128x128x2: the persistent two-stage kernel, one and two blocks per CU
 constexpr TileCost kTileCost[] = {
-    {64, 64, 3.288, 0.153, 0.184, 0.561, 0.027, 1.501},
-    {64, 128, 3.824, 0.261, 0.000, 0.001, 0.033, 2.355},
-    {128, 128, 0.434, 0.305, 4.394, 3.868, 0.168, 3.480},
-    {128, 256, 0.000, 0.463, 7.835, 6.446, 0.186, 3.150},
-    {256, 256, 2.954, 1.303, 5.631, 5.373, 0.169, 21.205},
+    {64, 64, 2.032, 0.119, 0.030, 0.030, 0.926, 0.143,
+     {0.357, 0.586, 0.000, 0.650, 0.298}, {0.024, 0.220, 0.711, 0.000, 0.000}},
+    {64, 128, 2.179, 0.197, 0.011, 0.065, 0.652, 0.168,
+     {0.042, 0.647, 0.528, 0.876, 0.000}, {0.427, 0.473, 1.345, 0.000, 0.160}},
+    {128, 128, 1.399, 0.290, 0.000, 0.179, 0.000, 0.548,
+     {2.022, 2.753, 1.857, 3.500, 2.059}, {0.548, 1.542, 4.708, 0.000, 0.000}},
+    {128, 256, 1.641, 0.390, 0.000, 0.412, 0.000, 1.180,
+     {2.282, 4.191, 2.899, 5.930, 2.662}, {1.698, 2.540, 7.192, 0.000, 0.000}},
+    {256, 256, 2.722, 1.090, 0.000, 0.593, 0.000, 0.000,
+     {2.974, 5.935, 4.000, 7.976, 2.672}, {2.436, 4.503, 15.553, 0.000, 0.288}},
+    {128, 128, 2.761, 0.028, 0.404, 0.214, 0.593, 0.000,
+     {0.780, 2.537, 1.700, 2.499, 0.401}, {0.223, 0.048, 2.379, 0.000, 0.213}},
 };
-// a consumer of norm partials on 256 x 256 tiles needs the row_rstd launch
-constexpr double kRowFactorLaunch = 4.5;
-Tile pick_tile(int64_t M, int64_t N, int64_t K, bool resid, bool norm) {
+static_assert(EPI_BF16 == 0 && EPI_F32 == 1 && EPI_RESID_F32 == 2 && EPI_QKV_ROPE == 3 &&
+                  EPI_SILU_GATE == 4, "kTileCost's epilogue columns");
+// a consumer of norm partials on the persistent tiles needs the row_rstd launch
+constexpr double kRowFactorLaunch = 3.4;
+bool takes_norm_partials(Tile t) { return t != T256x256 && t != T128x128x2; }
+Tile pick_tile(int64_t M, int64_t N, int64_t K, int epi, bool norm) {
   const int cus = device_cus() > 0 ? device_cus() : 256;
   const double KT = (double)(K / 64);
   const int64_t nb256 = ((M + 255) / 256) * (N / 256);
   if (nb256 >= 4 * (int64_t)cus) return T256x256;  // its rounds fill the chip
+  // the persistent tile with at least a block per CU; within the fit's error it is
+  // kept, since it moves the fewest operand bytes
+  const Tile persistent = nb256 < cus ? T128x128x2 : T256x256;
   double best = 0;
   Tile t = T256x256;
-  for (int i = 0; i < 5; ++i) {
+  for (int i = 0; i < 6; ++i) {
+    if (i == T128x128x2 && epi == EPI_QKV_ROPE) continue;  // (never the least)
     const TileCost& w = kTileCost[i];
     const int64_t n = ((M + w.bm - 1) / w.bm) * ((N + w.bn - 1) / w.bn);
-    const double c = (double)((n + cus - 1) / cus), f = (double)n / cus;
-    double est = w.fix + c * (w.k * KT + (resid ? w.e_resid : w.e_other)) +
-                 f * (w.kf * KT + (resid ? w.r : 0.0));
-    if (i == T256x256 && norm) est += kRowFactorLaunch;
-    // a full chip of 256 x 256 tiles moves the fewest operand bytes: leave it
-    // only for a clear gain
-    if (i == T256x256 && nb256 >= cus) est *= 0.95;
+    const double f = (double)n / cus, c1 = (double)((n + cus - 1) / cus),
+                 c2 = (double)((n + 2 * cus - 1) / (2 * cus));
+    double est = w.fix + (w.k1 * c1 + w.k2 * c2 + w.kf * f) * KT + w.e[epi] * c1 + w.o * c2 +
+                 w.r[epi] * f;
+    if (norm) est += takes_norm_partials((Tile)i) ? w.norm * f : kRowFactorLaunch;
+    if (i == persistent) est *= 0.97;
     if (i == 0 || est < best) {
       best = est;
       t = (Tile)i;
@@ -147,9 +172,13 @@ int run_gemm(const GemmArgs& a, hipStream_t s) {
 }  // namespace
 
 // (dense operands: the model's launches)
-bool gemm_takes_norm_partials(int64_t M, int64_t N, int64_t K, int np) {
+bool gemm_takes_norm_partials(int64_t M, int64_t N, int64_t K, int epi, int np) {
   return np % 4 == 0 && np <= 16 && N % 256 == 0 && K * 512 + K * 2 < (int64_t(1) << 31) &&
-         N * 1024 < (int64_t(1) << 31) && pick_tile(M, N, K, false, true) != T256x256;
+         N * 1024 < (int64_t(1) << 31) && takes_norm_partials(pick_tile(M, N, K, epi, true));
+}
+
+int gemm_tile(int64_t M, int64_t N, int64_t K, int epi) {
+  return N % 256 == 0 ? pick_tile(M, N, K, epi, false) : -1;
 }
 
 int launch_gemm(const GemmArgs& a_in, hipStream_t s) {
@@ -181,15 +210,17 @@ int launch_gemm(const GemmArgs& a_in, hipStream_t s) {
   // tile pick_tile chooses.  Otherwise (the 260-wide head, huge strides)
   // 128x128 register-staged tiles over 4 waves.
   if (a.N % 256 == 0 && tile_reach_fits(a)) {
-    switch (pick_tile(a.M, a.N, a.K, a.epi == EPI_RESID_F32, a.row_ss != nullptr)) {
+    const Tile t = pick_tile(a.M, a.N, a.K, a.epi, a.row_ss != nullptr);
+    if (a.row_ss && !takes_norm_partials(t))
+      return fail(-2, "gemm: this launch does not take norm partials");
+    switch (t) {
       case T64x64: return run_gemm_pipe_epi<64, 64, 2, 1, 2, 5>(a, s);
       case T64x128: return run_gemm_pipe_epi<64, 128, 2, 2, 4, 3>(a, s);
       case T128x128: return run_gemm_pipe_epi<128, 128, 4, 2, 4, 5>(a, s);
       case T128x256: return run_gemm_pipe_epi<128, 256, 2, 4, 4, 3>(a, s);
-      case T256x256: break;
+      case T128x128x2: return run_gemm_dma_epi<128, 128, 64, 2, 2>(a, s);
+      case T256x256: return run_gemm_dma_epi<256, 256, 64, 2, 4>(a, s);
     }
-    if (a.row_ss) return fail(-2, "gemm: this launch does not take norm partials");
-    return run_gemm_dma_epi<256, 256, 64, 2, 4>(a, s);
   }
   if (a.row_ss) return fail(-2, "gemm: this launch does not take norm partials");
   return run_gemm<128, 128, 32, 2, 2, 2, 3>(a, s);

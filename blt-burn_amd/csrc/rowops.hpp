@@ -128,9 +128,11 @@ struct GemmArgs {
   int row_np, row_dim;
   float row_eps;
 };
-// whether a (non-residual) launch of this shape with np norm partials per row
-// forms the row factors itself (row_ss); otherwise it needs row_scale
-bool gemm_takes_norm_partials(int64_t M, int64_t N, int64_t K, int np);
+// whether a launch of this shape with np norm partials per row forms the row
+// factors itself (row_ss); otherwise it needs row_scale
+bool gemm_takes_norm_partials(int64_t M, int64_t N, int64_t K, int epi, int np);
+// the tile of a launch with dense operands (blt_gemm_tile)
+int gemm_tile(int64_t M, int64_t N, int64_t K, int epi);
 int launch_gemm(const GemmArgs& a, hipStream_t s);
 
 // k_attn.hip -----------------------------------------------------------------

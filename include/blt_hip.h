@@ -527,6 +527,12 @@ int blt_gemm_bf16_epilogue(const uint16_t* A, const uint16_t* Bt, void* C, int64
                            int32_t n_valid, int32_t rope_cols, int64_t seq_len,
                            const float* rope_cs, blt_stream_t stream);
 
+/* The tile that such a launch with dense operands takes on the current GPU (256 CUs
+ * where there is none): 0 .. 3 = 64x64, 64x128, 128x128, 128x256 (one block per
+ * tile), 4 = 256x256, 5 = 128x128 (persistent blocks), -1 = register-staged (N % 256
+ * != 0); -2 on bad arguments.  Launches nothing; for tests and tuning. */
+int32_t blt_gemm_tile(int64_t M, int64_t N, int64_t K, int32_t epilogue);
+
 /* Measurement helpers (no counterpart in the reference; bench.py reads the
  * rates this GPU sustains beside the published peaks) --------------------- */
 

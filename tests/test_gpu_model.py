@@ -15,7 +15,7 @@ import torch
 import np_ref
 import oracle
 from blt_burn_amd import model as M
-from blt_burn_amd import patcher, synth
+from blt_burn_amd import _lib, patcher, synth
 
 pytestmark = pytest.mark.gpu
 
@@ -106,9 +106,13 @@ def _far_norm_weights(cfg, seed, hidden):
 
 @pytest.mark.parametrize("B,T", [(1, 1), (1, 2), (3, 3), (2, 33)])
 def test_entropy_model_few_tokens(B, T):
-    # a handful of tokens at real size: every projection runs on 128 x 128
-    # tiles that are almost all padding rows, attention on one partial key
+    # a handful of tokens at real size: every projection runs on 64 x 64 tiles
+    # (asserted) that are almost all padding rows, attention on one partial key
     # tile, the boundary pass on its T <= 2 special cases
+    tile = _lib.lib().blt_gemm_tile
+    for N, K, epi in ((2304, 768, _lib.EPI_QKV_ROPE), (768, 768, _lib.EPI_RESID_F32),
+                      (4096, 768, _lib.EPI_SILU_GATE), (768, 2048, _lib.EPI_RESID_F32)):
+        assert tile(B * T, N, K, epi) == 0
     cfg = M.entropy_model_config()
     out, ref = _run(cfg, 2048, B, T, 512, seed=6)
     _compare(out, ref, "entropy-model B=%d T=%d" % (B, T))

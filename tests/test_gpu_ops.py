@@ -676,12 +676,12 @@ def test_gemm_f32_epilogue_partial_columns(M, N):
 @pytest.mark.parametrize("K", [192, 768])
 @pytest.mark.parametrize("epi", ["bf16", "resid", "f32", "silu", "qkv"])
 def test_gemm_small_launch_tiles_bit_identical(epi, K):
-    # A launch with fewer 256 x 256 tiles than CUs runs on 128 x 128 tiles; its
-    # rows must equal the same rows of a launch that stays on 256 x 256 tiles,
-    # bit for bit (the model's row-independence rests on it), also on the
-    # column blocks whose K tiles run from the last one down (N > 1024).
-    Mb, Ms = 256 * 256 + 64, 1000
+    # A launch with far fewer 256 x 256 tiles than CUs runs on smaller tiles;
+    # its rows must equal the same rows of a launch on 256 x 256 tiles, bit for
+    # bit (the model's row-independence rests on it), also on the column blocks
+    # whose K tiles run from the last one down (N > 1024).
     N = {"silu": 4096, "qkv": 2304}.get(epi, 768)
+    Mb, Ms = 256 * -(-1024 // (N // 256)) + 64, 1000
     torch.manual_seed(5)
     a = torch.randn(Mb, K, device=DEV).to(torch.bfloat16)
     bt = (0.05 * torch.randn(N, K, device=DEV)).to(torch.bfloat16)
@@ -694,6 +694,8 @@ def test_gemm_small_launch_tiles_bit_identical(epi, K):
         kw = dict(n_valid=N)
     code = {"bf16": _lib.EPI_BF16, "resid": _lib.EPI_RESID_F32, "f32": _lib.EPI_F32,
             "silu": _lib.EPI_SILU_GATE, "qkv": _lib.EPI_QKV_ROPE}[epi]
+    tile = _lib.lib().blt_gemm_tile
+    assert tile(Mb, N, K, code) == 4 and tile(Ms, N, K, code) in (0, 1, 2, 3)
     if epi in ("resid", "f32"):
         big = torch.randn(Mb, N, device=DEV)
     else:
@@ -705,9 +707,11 @@ def test_gemm_small_launch_tiles_bit_identical(epi, K):
 
 
 # Every tile the launch selection picks between (64 x 64 up to 128 x 256, one
-# block per tile with loader waves) at the edges of its row tiles, with K tiles
-# fewer than, equal to and more than the stages: bit-identical to the same rows
-# of a 256 x 256 launch.
+# block per tile with loader waves; 128 x 128 on persistent blocks) at the edges
+# of its row tiles, with K tiles fewer than, equal to and more than the stages:
+# bit-identical to the same rows of a 256 x 256 launch.  Row counts are added
+# until every tile that any of them leads to has been run; K = 2048 leads to all
+# four small ones with every epilogue.
 @pytest.mark.parametrize("K", [64, 256, 320, 2048])
 @pytest.mark.parametrize("epi", ["bf16", "resid", "f32", "silu", "qkv"])
 def test_gemm_every_launch_tile_bit_identical(epi, K):
@@ -732,8 +736,17 @@ def test_gemm_every_launch_tile_bit_identical(epi, K):
     big = base.clone()
     _gemm_epi(a, bt, big, code, **kw)
     guard = 70  # rows past M stay as they are
-    for M in (1, 31, 33, 63, 65, 127, 129, 300, 513, 1000, 1500, 2100, 2561, 3100, 4200, 5121,
-              6150, 8200, 10300):
+    tile = lambda M: _lib.lib().blt_gemm_tile(M, N, K, code)
+    assert tile(Mb) == 4
+    Ms = [1, 31, 33, 63, 65, 127, 129, 300, 513, 1000, 1500, 2100, 2561, 3100, 4200, 5121, 6150,
+          8200, 10300]
+    first = {}
+    for M in list(range(19, Mb - guard, 131)):
+        first.setdefault(tile(M), M)
+    Ms += [M for t, M in first.items() if t not in map(tile, Ms)]
+    run = set(map(tile, Ms))
+    assert run >= ({0, 1, 2, 3, 4} if K == 2048 else {4}) and run >= set(first), run
+    for M in Ms:
         small = base[:M + guard].clone()
         _gemm_epi(a[:M].contiguous(), bt, small[:M], code, **kw)
         assert torch.equal(small[:M], big[:M]), M
