@@ -674,7 +674,7 @@ int Ingest::run(const int32_t* tokens, const int64_t* doc_off, int64_t n_docs, f
     const int64_t nd = (int64_t)s.units.size();
     const int64_t longest = nd > 0 ? *std::max_element(s.h_dlen, s.h_dlen + nd) : 0;
     stats.batches += 1;
-    stats.row_tokens += BT;
+    stats.row_tokens += Mu;
     // ---- upload ----
     const size_t ub = (size_t)Mu * 4;
     BLT_HIP_CHECK(hipMemcpyAsync(s.d_tok, s.h_tok, ub, hipMemcpyHostToDevice, up));

@@ -165,7 +165,8 @@ class StreamingIngest:
 
     def last_stats(self):
         """Counts of the last run(): dict(batches, documents, tokens, tokens_computed,
-        row_tokens)."""
+        row_tokens): row_tokens is the packed-row slots that were run, padding
+        included."""
         st = IngestStats()
         check(_lib.lib().blt_ingest_last_stats(self._h, ctypes.byref(st)), "ingest_last_stats")
         return {n: int(getattr(st, n)) for n, _ in IngestStats._fields_}

@@ -407,9 +407,10 @@ int blt_ingest_run_patch_means(blt_ingest* g, const int32_t* tokens, const int64
                                int32_t* counts, float* patch_entropy, float* patch_prominence,
                                float* patch_coherence);
 /* Counts of the last blt_ingest_run: non-empty documents and their tokens,
- * tokens run through the model (chunks, overlap context included) and the
- * batches' packed-row slots (batches * rows * row_len, padding included; the
- * unused rows of a batch, and the unused end of its rows, are not run). */
+ * tokens run through the model (chunks, overlap context included) and
+ * packed-row slots launched (padding included; a batch launches its used rows,
+ * cut to their longest fill where a sixteenth of every row is free, so at most
+ * batches * rows * row_len). */
 typedef struct blt_ingest_stats {
   int64_t batches;
   int64_t documents;
