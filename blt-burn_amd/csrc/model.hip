@@ -278,7 +278,7 @@ int Model::forward(const int32_t* tokens, int64_t B, int64_t T, const blt_model_
     return rc;
   const int np = (int)(D / 64);
   // Small launches form the row factors from the norm partials themselves (a
-  // row_rstd launch is about 4.5 us of dependency latency, twice per layer);
+  // row_rstd launch is 3 to 4.5 us of dependency latency, twice per layer);
   // on the persistent tiles those scattered loads cost more than the launch.
   const bool qkv_ss = carry && gemm_takes_norm_partials(M, 3 * D, D, EPI_QKV_ROPE, np);
   const bool w13_ss = carry && gemm_takes_norm_partials(M, 2 * F, D, EPI_SILU_GATE, np);
