@@ -463,8 +463,9 @@ int run_attention(const AttnArgs& a, hipStream_t s) {
 // B = 4, H = 12, T = 2048, d = 64, full 6720 -> 590 (87 TFLOP/s); B = 1, H = 4, T
 // = 2048, d = 128, causal 2310 -> 78.  Without its K and V loads the full case
 // takes 390 us: what is left is the loads, K's 32 rows x 32 bytes per
-// instruction above all.  The largest error against 64 bits is no larger than
-// the VALU kernel's (2.0e-7 against 3.2e-7 rel on the first case).
+// instruction above all.  Error against 64 bits: 2.0e-7 rel on the first case, where
+// the VALU kernel had 3.2e-7; over seeds of ten shapes (1 to 1500 keys, d = 32 .. 128)
+// the mean is 0.53 to 0.91 of that kernel's, least with many keys.
 constexpr int F_MAXD = 256;
 
 // ROW: how rows are read: 2 = d is 32 ND and every tensor 16-byte aligned; 1 = d % 4
